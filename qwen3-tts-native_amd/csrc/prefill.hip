@@ -378,6 +378,7 @@ hipError_t launch_bf16_gemm(const Bf16GemmArgs& g, hipStream_t stream) {
     }
     const uintptr_t align = reinterpret_cast<uintptr_t>(g.a) | reinterpret_cast<uintptr_t>(g.b);
     if ((align & 15u) != 0 || (g.a_batch % 8) != 0 || (g.b_batch % 8) != 0) return hipErrorInvalidValue;
+    if (gemm_dma_takes(g)) return launch_gemm_dma(g, stream);
     // Tiles, K steps and K slices, measured on MI355X over the prefill's
     // shapes (prompts of 16..801 rows, N 1024..6144, K 2048 / 6144): 128-square
     // only where it still gives two workgroups per CU; else 32-square up to

@@ -447,7 +447,11 @@ hipError_t launch_sum_embeddings(const bf16_t* const* tables, int count, int voc
 // Epilogues of the bf16 GEMM: C = bf16(sum); C = bf16(C + bf16(sum)) (the
 // residual add_in_place); C = bf16(bf16(silu(C)) * bf16(sum)) (silu_gate with
 // C holding the gate product).
-enum Bf16GemmEpilogue : int { kGemmStore = 0, kGemmAddInto = 1, kGemmSiluGateInto = 2 };
+enum Bf16GemmEpilogue : int {
+    kGemmStore = 0,
+    kGemmAddInto = 1,
+    kGemmSiluGateInto = 2,
+};
 
 struct Bf16GemmArgs {
     const bf16_t* a = nullptr;
@@ -474,6 +478,13 @@ struct Bf16GemmArgs {
     int b2_row = 0, b3_row = 0;
 };
 hipError_t launch_bf16_gemm(const Bf16GemmArgs& args, hipStream_t stream);
+// The same products through direct-to-LDS loads (gemm_dma.hip): unbatched, K a
+// multiple of 64, planned.  launch_bf16_gemm runs them where they are taken.
+bool gemm_dma_takes(const Bf16GemmArgs& args);
+hipError_t launch_gemm_dma(const Bf16GemmArgs& args, hipStream_t stream);
+// C = silu_gate(bf16(A b^T), bf16(A b2^T)), both products in one launch: b the
+// gate's, b2 the up projection's [n][k] weights (taken as above).
+hipError_t launch_gate_up_gemm(const Bf16GemmArgs& args, hipStream_t stream);
 // Prompts of at most this many positions run the reference's GEMM attention
 // (scores materialized, causal softmax); longer ones the exact per-row kernel
 // (talker.cu:3035-3054 with kPrefillGemmCapacity = 512).

@@ -848,9 +848,20 @@ public:
             // O GEMM with the residual add (add_in_place) as its epilogue
             gemm(attn, qw, L.o16, hidden, H, H, qw, "prefill O GEMM + residual", kGemmAddInto);
             check_hip(launch_rms_norm_rows(hidden, L.post_norm, xn, rows, H, cfg_.eps, stream_), "prefill post norm");
-            gemm(xn, H, L.gate16, gate, I, I, H, "prefill gate GEMM");
-            // up GEMM with silu_gate as its epilogue (gate holds the gate product)
-            gemm(xn, H, L.up16, gate, I, I, H, "prefill up GEMM + SiLU gate", kGemmSiluGateInto);
+            {  // gate and up GEMMs in one launch, silu_gate as their epilogue
+                Bf16GemmArgs g;
+                g.a = xn;
+                g.b = L.gate16;
+                g.b2 = L.up16;
+                g.c = gate;
+                g.m = rows;
+                g.n = I;
+                g.k = H;
+                g.lda = H;
+                g.ldb = H;
+                g.ldc = I;
+                check_hip(launch_gate_up_gemm(g, stream_), "prefill gate/up GEMM + SiLU gate");
+            }
             gemm(gate, I, L.down16, hidden, H, H, I, "prefill down GEMM + residual", kGemmAddInto);
         }
     }
