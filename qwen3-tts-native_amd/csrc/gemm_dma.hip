@@ -54,8 +54,8 @@ __device__ __forceinline__ void wait_and_sync() {
 constexpr int kGemmGated = 16;
 
 // Four consecutive columns of one row.  Rounding as the separate launches':
-// the product to bf16, then the residual add or silu_gate over the gate product
-// in C.
+// the product to bf16, then the residual add, silu_gate over the gate product
+// in C, or the bias (with the text projection's scale and SiLU).
 template <int kEpilogue>
 __device__ __forceinline__ void store4(const Bf16GemmArgs& g, int row, int col, const floatx4_t& v) {
     bf16_t* out = g.c + static_cast<size_t>(row) * g.ldc + col;
@@ -76,6 +76,18 @@ __device__ __forceinline__ void store4(const Bf16GemmArgs& g, int row, int col, 
         r.y = one(o.y, v[1]);
         r.z = one(o.z, v[2]);
         r.w = one(o.w, v[3]);
+    } else if constexpr (kEpilogue == kGemmScaleBias || kEpilogue == kGemmScaleBiasSilu) {
+        const float4 s = *reinterpret_cast<const float4*>(g.scales + col);
+        const ushort4 b = *reinterpret_cast<const ushort4*>(g.bias + col);
+        auto one = [](float x, bf16_t bias) {
+            float y = round_bf(x) + bf2f(bias);
+            if constexpr (kEpilogue == kGemmScaleBiasSilu) y *= 1.0f / (1.0f + q3_expf(-y));
+            return f2bf(y);
+        };
+        r.x = one(v[0] * s.x, b.x);
+        r.y = one(v[1] * s.y, b.y);
+        r.z = one(v[2] * s.z, b.z);
+        r.w = one(v[3] * s.w, b.w);
     } else {
         r.x = f2bf(v[0]);
         r.y = f2bf(v[1]);
@@ -380,7 +392,8 @@ bool gemm_dma_takes(const Bf16GemmArgs& g) {
     if (!aligned(g.a, 16) || !aligned(g.b, 16) || !aligned(g.b2, 16) || !aligned(g.b3, 16) || !aligned(g.c, 8)) return false;
     if (g.partial != nullptr && !aligned(g.partial, 16)) return false;
     if (static_cast<long long>(g.m) * g.n > (1LL << 31) - 1) return false;
-    return true;
+    const bool biased = g.epilogue == kGemmScaleBias || g.epilogue == kGemmScaleBiasSilu;
+    return !biased || (g.scales != nullptr && g.bias != nullptr && aligned(g.scales, 16) && aligned(g.bias, 8));
 }
 
 hipError_t launch_gemm_dma(const Bf16GemmArgs& g, hipStream_t stream) {
@@ -389,6 +402,8 @@ hipError_t launch_gemm_dma(const Bf16GemmArgs& g, hipStream_t stream) {
         case kGemmStore: return launch_plain<kGemmStore>(g, stream);
         case kGemmAddInto: return launch_plain<kGemmAddInto>(g, stream);
         case kGemmSiluGateInto: return launch_plain<kGemmSiluGateInto>(g, stream);
+        case kGemmScaleBias: return launch_plain<kGemmScaleBias>(g, stream);
+        case kGemmScaleBiasSilu: return launch_plain<kGemmScaleBiasSilu>(g, stream);
         default: return hipErrorInvalidValue;
     }
 }

@@ -936,47 +936,6 @@ hipError_t launch_int8_gemv(const GemvArgs& a, hipStream_t stream) {
     }
 }
 
-// A prompt's rows (any count) in exact order through one launch, each row's
-// result the same as through launch_int8_gemv in launches of up to 8 rows
-// (the per-row sum does not depend on the rows beside it).  No RMSNorm
-// prologue; store and bias epilogues; K outside {1024, 2048, 3072, 6144} runs
-// as launches of up to 8 rows.
-hipError_t launch_int8_gemv_prompt_rows(const GemvArgs& a, hipStream_t stream) {
-    if (a.weight == nullptr || a.scales == nullptr || a.input == nullptr || a.out16 == nullptr || a.rows < 1 ||
-        a.out_features <= 0 || a.norm_weight != nullptr || a.input_row_index != nullptr || a.out32 != nullptr ||
-        !aligned16(a.weight) || !aligned16(a.input)) {
-        return hipErrorInvalidValue;
-    }
-    if (a.epilogue >= kEpiBias && a.bias == nullptr) return hipErrorInvalidValue;
-    auto by_k = [&](auto epi) -> hipError_t {
-        constexpr int kE = decltype(epi)::value;
-        switch (a.in_features) {
-            case 1024: return launch_exact_rows_fixed<2, kE>(a, stream);
-            case 2048: return launch_exact_rows_fixed<4, kE>(a, stream);
-            case 3072: return launch_exact_rows_fixed<6, kE>(a, stream);
-            case 6144: return launch_exact_rows_fixed<12, kE>(a, stream);
-            default: break;
-        }
-        // other widths: launches of up to 8 rows
-        for (int r0 = 0; r0 < a.rows; r0 += 8) {
-            GemvArgs part = a;
-            part.rows = std::min(8, a.rows - r0);
-            part.mode = kModeExact;
-            part.input = a.input + static_cast<size_t>(r0) * a.in_features;
-            part.out16 = a.out16 + static_cast<size_t>(r0) * a.out_features;
-            const hipError_t st = launch_int8_gemv(part, stream);
-            if (st != hipSuccess) return st;
-        }
-        return hipSuccess;
-    };
-    switch (a.epilogue) {
-        case kEpiStore: return by_k(std::integral_constant<int, kEpiStore>{});
-        case kEpiBias: return by_k(std::integral_constant<int, kEpiBias>{});
-        case kEpiBiasSilu: return by_k(std::integral_constant<int, kEpiBiasSilu>{});
-        default: return hipErrorInvalidValue;
-    }
-}
-
 hipError_t launch_quantize_weight_rows(const bf16_t* weight, int8_t* quantized, float* scales,
                                        int in_features, int out_features, hipStream_t stream) {
     if (in_features % 16 != 0 || in_features <= 0 || out_features <= 0) return hipErrorInvalidValue;

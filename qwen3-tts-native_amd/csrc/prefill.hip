@@ -359,7 +359,22 @@ __global__ __launch_bounds__(256) void gather_text_rows_kernel(const bf16_t* tab
     }
 }
 
+__global__ __launch_bounds__(256) void int8_to_bf16_kernel(const int8_t* source, bf16_t* destination, size_t groups) {
+    const size_t t = static_cast<size_t>(blockIdx.x) * 256 + threadIdx.x;
+    if (t >= groups) return;
+    const int8_t* s = source + t * 8;
+    bf16_t* d = destination + t * 8;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) d[i] = f2bf(static_cast<float>(s[i]));
+}
+
 }  // namespace
+
+hipError_t launch_int8_to_bf16(const int8_t* source, bf16_t* destination, size_t count, hipStream_t stream) {
+    if (source == nullptr || destination == nullptr || count == 0 || count % 8 != 0) return hipErrorInvalidValue;
+    int8_to_bf16_kernel<<<static_cast<unsigned>((count / 8 + 255) / 256), 256, 0, stream>>>(source, destination, count / 8);
+    return hipGetLastError();
+}
 
 hipError_t launch_bf16_gemm(const Bf16GemmArgs& g, hipStream_t stream) {
     if (g.a == nullptr || g.b == nullptr || g.c == nullptr || g.m <= 0 || g.n <= 0 || g.k <= 0 || g.batch <= 0 ||

@@ -254,9 +254,6 @@ private:
     hipStream_t stream_ = nullptr;
     hipError_t status_ = hipSuccess;
 };
-// Exact-order rows of a prompt (any count, no RMSNorm) in one launch.
-hipError_t launch_int8_gemv_prompt_rows(const GemvArgs& a, hipStream_t stream);
-
 hipError_t launch_quantize_weight_rows(const bf16_t* weight, int8_t* quantized, float* scales,
                                        int in_features, int out_features, hipStream_t stream);
 hipError_t launch_int8_gemm_rows(const int8_t* weight, const float* scales, const bf16_t* input,
@@ -446,11 +443,14 @@ hipError_t launch_sum_embeddings(const bf16_t* const* tables, int count, int voc
 // ldb, a_batch and b_batch must be multiples of 8 and A, B 16-byte aligned.
 // Epilogues of the bf16 GEMM: C = bf16(sum); C = bf16(C + bf16(sum)) (the
 // residual add_in_place); C = bf16(bf16(silu(C)) * bf16(sum)) (silu_gate with
-// C holding the gate product).
+// C holding the gate product); C = bf16(bf16(sum * scale[n]) + bias[n]), plain
+// and with SiLU (the text projection over its int8 weights as bf16 integers).
 enum Bf16GemmEpilogue : int {
     kGemmStore = 0,
     kGemmAddInto = 1,
     kGemmSiluGateInto = 2,
+    kGemmScaleBias = 3,
+    kGemmScaleBiasSilu = 4,
 };
 
 struct Bf16GemmArgs {
@@ -476,6 +476,8 @@ struct Bf16GemmArgs {
     const bf16_t* b2 = nullptr;
     const bf16_t* b3 = nullptr;
     int b2_row = 0, b3_row = 0;
+    const float* scales = nullptr;   // kGemmScaleBias*: per column
+    const bf16_t* bias = nullptr;
 };
 hipError_t launch_bf16_gemm(const Bf16GemmArgs& args, hipStream_t stream);
 // The same products through direct-to-LDS loads (gemm_dma.hip): unbatched, K a
@@ -496,6 +498,8 @@ hipError_t launch_prefill_qkv_epilogue(bf16_t* qkv, const bf16_t* q_norm, const 
                                        int query_heads, int key_value_heads, float epsilon, hipStream_t stream);
 hipError_t launch_transpose_values(const bf16_t* qkv, int qkv_width, int v_offset, int rows, int stride,
                                    int key_value_heads, bf16_t* vt, hipStream_t stream);
+// Integers as bf16 (exact: |v| <= 127); count a multiple of 8.
+hipError_t launch_int8_to_bf16(const int8_t* source, bf16_t* destination, size_t count, hipStream_t stream);
 hipError_t launch_prompt_rows(bf16_t* rows_data, const int* text, const int* codec, const bf16_t* codec_embedding,
                               int codec_vocabulary, int rows, int width, hipStream_t stream);
 hipError_t launch_gather_text_rows(const bf16_t* table, const int* text, int vocabulary, int rows, int width,

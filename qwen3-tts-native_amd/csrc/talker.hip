@@ -392,6 +392,12 @@ public:
         };
         text_fc1_ = qt(fc1_off);
         text_fc2_ = qt(fc2_off);
+        // the text projection's integers as bf16 for the prompt's GEMMs
+        const size_t text_elements = static_cast<size_t>(T.hidden) * T.hidden;
+        text16_ = DeviceBuffer(2 * text_elements * sizeof(bf16_t));
+        check_hip(launch_int8_to_bf16(text_fc1_.data, text16_.as<bf16_t>(), text_elements, upload_stream_), "text fc1 as bf16");
+        check_hip(launch_int8_to_bf16(text_fc2_.data, text16_.as<bf16_t>() + text_elements, text_elements, upload_stream_),
+                  "text fc2 as bf16");
         small_to_mtp_ = qt(small_off);
         codec_head_ = qt(codec_head_off);
         for (int g = 0; g < kResidualCodebooks; ++g) predictor_heads_[g] = qt(head_off[g]);
@@ -456,7 +462,7 @@ private:
     size_t int8_bytes_ = 0;
     hipStream_t upload_stream_ = nullptr;
     std::unordered_map<std::string, DeviceTensor> tensors_;
-    DeviceBuffer int8_arena_, scale_arena_, embedding_tables_, rope_table_;
+    DeviceBuffer int8_arena_, scale_arena_, text16_, embedding_tables_, rope_table_;
     std::vector<Layer> talker_layers_, predictor_layers_;
     QTensor text_fc1_, text_fc2_, small_to_mtp_, codec_head_;
     const bf16_t* codec_head16_ = nullptr;
@@ -512,7 +518,6 @@ struct Gemv {
         return *this;
     }
     void run(hipStream_t s, const char* what) { check_hip(launch_int8_gemv(a, s), what); }
-    void run_prompt_rows(hipStream_t s, const char* what) { check_hip(launch_int8_gemv_prompt_rows(a, s), what); }
 };
 
 struct SamplingParams {
@@ -729,17 +734,34 @@ public:
         w.ensure(rows, H, I, qkvw, qw, T.query_heads, T.key_value_heads, gemm_attention ? rp : 0,
                  gemm_attention ? 0 : max_seq_);
         bf16_t* hidden = w.hidden.as<bf16_t>();
-        // prompt embeddings: int8 text projection (exact order, 8 rows a
-        // launch), then zero text-less rows and add codec embeddings
+        // prompt embeddings: int8 text projection, then zero text-less rows
+        // and add codec embeddings.  The integers run as bf16 (exactly) on the
+        // matrix cores, scale and bias in the epilogue: the same products
+        // summed in fp32, in another order than the decode step's GEMVs
+        // (512 rows: 318 us as exact-order GEMVs, 35 us here).
         check_hip(launch_gather_text_rows(m_.text_embedding_, text_ids, cfg_.text_vocab, rows, H, w.normalized.as<bf16_t>(),
                                           stream_),
                   "gather prompt text embeddings");
-        // (the reference runs 8 rows a launch; each row's exact-order sum is
-        // the same whatever rows share its launch, so all rows run in one)
-        Gemv(m_.text_fc1_, w.normalized.as<bf16_t>(), H, H, kEpiBiasSilu).bias(m_.text_fc1_bias_)
-            .rows(rows, kModeExact).to(w.proj.as<bf16_t>()).run_prompt_rows(stream_, "prompt text fc1");
-        Gemv(m_.text_fc2_, w.proj.as<bf16_t>(), H, H, kEpiBias).bias(m_.text_fc2_bias_)
-            .rows(rows, kModeExact).to(hidden).run_prompt_rows(stream_, "prompt text fc2");
+        const bf16_t* fc16 = m_.text16_.as<bf16_t>();
+        Bf16GemmArgs fc;
+        fc.a = w.normalized.as<bf16_t>();
+        fc.b = fc16;
+        fc.c = w.proj.as<bf16_t>();
+        fc.m = rows;
+        fc.n = fc.k = fc.lda = fc.ldb = fc.ldc = H;
+        fc.partial = w.partial.as<float>();
+        fc.partial_floats = kPrefillPartialFloats;
+        fc.epilogue = kGemmScaleBiasSilu;
+        fc.scales = m_.text_fc1_.scales;
+        fc.bias = m_.text_fc1_bias_;
+        check_hip(launch_gemm_dma(fc, stream_), "prompt text fc1");
+        fc.a = w.proj.as<bf16_t>();
+        fc.b = fc16 + static_cast<size_t>(H) * H;
+        fc.c = hidden;
+        fc.epilogue = kGemmScaleBias;
+        fc.scales = m_.text_fc2_.scales;
+        fc.bias = m_.text_fc2_bias_;
+        check_hip(launch_gemm_dma(fc, stream_), "prompt text fc2");
         check_hip(launch_prompt_rows(hidden, text_ids, codec_ids, m_.codec_embedding_, cfg_.talker_vocab, rows, H, stream_),
                   "prompt rows");
         auto gemm = [&](const bf16_t* a, int lda, const bf16_t* weight, bf16_t* c, int ldc, int n, int k,
