@@ -318,18 +318,6 @@ __global__ __launch_bounds__(64) void prefill_qkv_epilogue_kernel(bf16_t* qkv, c
     }
 }
 
-// vt[h][d][j] = v(row j, head h, dim d) for j < rows, 0 for rows <= j < stride.
-__global__ __launch_bounds__(256) void transpose_values_kernel(const bf16_t* qkv, int qkv_width, int v_offset, int rows,
-                                                               int stride, int key_value_heads, bf16_t* vt) {
-    const size_t total = static_cast<size_t>(key_value_heads) * 128 * stride;
-    for (size_t t = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x; t < total;
-         t += static_cast<size_t>(gridDim.x) * blockDim.x) {
-        const int j = static_cast<int>(t % stride);
-        const int hd = static_cast<int>(t / stride);  // h * 128 + d
-        vt[t] = j < rows ? qkv[static_cast<size_t>(j) * qkv_width + v_offset + hd] : f2bf(0.0f);
-    }
-}
-
 // Prompt rows: out[r] = (text[r] >= 0 ? projected[r] : 0), then + the codec
 // embedding of codec[r] when codec[r] >= 0 (bf16 add), as the reference's
 // prepare_prompt_embedding (talker.cu:2721-2748).
@@ -480,15 +468,6 @@ hipError_t launch_prefill_qkv_epilogue(bf16_t* qkv, const bf16_t* q_norm, const 
     prefill_qkv_epilogue_kernel<<<rows * heads, 64, 0, stream>>>(qkv, q_norm, k_norm, rope_table, key_cache, value_cache,
                                                                  value_stride, first, query_heads, key_value_heads,
                                                                  epsilon);
-    return hipGetLastError();
-}
-
-hipError_t launch_transpose_values(const bf16_t* qkv, int qkv_width, int v_offset, int rows, int stride,
-                                   int key_value_heads, bf16_t* vt, hipStream_t stream) {
-    if (rows <= 0 || stride < rows || key_value_heads <= 0) return hipErrorInvalidValue;
-    const size_t total = static_cast<size_t>(key_value_heads) * 128 * stride;
-    const int blocks = static_cast<int>(std::min<size_t>((total + 255) / 256, 4096));
-    transpose_values_kernel<<<blocks, 256, 0, stream>>>(qkv, qkv_width, v_offset, rows, stride, key_value_heads, vt);
     return hipGetLastError();
 }
 

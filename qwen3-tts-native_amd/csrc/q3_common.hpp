@@ -487,17 +487,19 @@ hipError_t launch_gemm_dma(const Bf16GemmArgs& args, hipStream_t stream);
 // C = silu_gate(bf16(A b^T), bf16(A b2^T)), both products in one launch: b the
 // gate's, b2 the up projection's [n][k] weights (taken as above).
 hipError_t launch_gate_up_gemm(const Bf16GemmArgs& args, hipStream_t stream);
-// Prompts of at most this many positions run the reference's GEMM attention
-// (scores materialized, causal softmax); longer ones the exact per-row kernel
-// (talker.cu:3035-3054 with kPrefillGemmCapacity = 512).
+// Rows that the causal softmax takes (the reference's materialized scores,
+// kPrefillGemmCapacity, talker.cu:3035-3054).
 constexpr int kPrefillAttentionRows = 512;
+// The prompt's causal attention (any number of rows): q rows of qkv against
+// the key cache [position][kv width] and the blocked value cache.
+hipError_t launch_prefill_attention(const bf16_t* qkv, int qkv_width, const bf16_t* key_cache, const bf16_t* value_cache,
+                                    int value_stride, bf16_t* out, int rows, int query_heads, int key_value_heads,
+                                    int head_dimension, hipStream_t stream);
 hipError_t launch_causal_softmax(bf16_t* scores, int heads, int rows, int stride, int head_dimension,
                                  hipStream_t stream);
 hipError_t launch_prefill_qkv_epilogue(bf16_t* qkv, const bf16_t* q_norm, const bf16_t* k_norm, const bf16_t* rope_table,
                                        bf16_t* key_cache, bf16_t* value_cache, int value_stride, int first, int rows,
                                        int query_heads, int key_value_heads, float epsilon, hipStream_t stream);
-hipError_t launch_transpose_values(const bf16_t* qkv, int qkv_width, int v_offset, int rows, int stride,
-                                   int key_value_heads, bf16_t* vt, hipStream_t stream);
 // Integers as bf16 (exact: |v| <= 127); count a multiple of 8.
 hipError_t launch_int8_to_bf16(const int8_t* source, bf16_t* destination, size_t count, hipStream_t stream);
 hipError_t launch_prompt_rows(bf16_t* rows_data, const int* text, const int* codec, const bf16_t* codec_embedding,

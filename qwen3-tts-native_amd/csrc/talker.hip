@@ -720,54 +720,17 @@ public:
 
     // The prompt's rows through the talker with the bf16 weights
     // (run_decoder_prefill, talker.cu:2854-3202): every projection one MFMA
-    // GEMM over all rows; attention through materialized scores and the
-    // causal softmax when the prompt fits kPrefillAttentionRows and the
-    // session capacity (talker.cu:3035), else the exact per-row kernel.
+    // GEMM over all rows, attention one launch over all rows and heads.
     // Leaves the rows' final hidden states in prefill_.hidden.
     void prefill_bf16(int rows, const int* text_ids, const int* codec_ids) {
         const Dims& T = cfg_.talker;
         const int H = T.hidden, I = T.intermediate, qw = T.query_width(), kvw = T.kv_width();
         const int qkvw = T.qkv_width(), hd = T.head_dimension;
-        const int rp = (rows + 7) / 8 * 8;
-        const bool gemm_attention = rows <= std::min(max_seq_, kPrefillAttentionRows);
         PrefillBuffers& w = prefill_;
-        w.ensure(rows, H, I, qkvw, qw, T.query_heads, T.key_value_heads, gemm_attention ? rp : 0,
-                 gemm_attention ? 0 : max_seq_);
+        w.ensure(rows, H, I, qkvw, qw);
         bf16_t* hidden = w.hidden.as<bf16_t>();
-        // prompt embeddings: int8 text projection, then zero text-less rows
-        // and add codec embeddings.  The integers run as bf16 (exactly) on the
-        // matrix cores, scale and bias in the epilogue: the same products
-        // summed in fp32, in another order than the decode step's GEMVs
-        // (512 rows: 318 us as exact-order GEMVs, 35 us here).
-        check_hip(launch_gather_text_rows(m_.text_embedding_, text_ids, cfg_.text_vocab, rows, H, w.normalized.as<bf16_t>(),
-                                          stream_),
-                  "gather prompt text embeddings");
-        const bf16_t* fc16 = m_.text16_.as<bf16_t>();
-        Bf16GemmArgs fc;
-        fc.a = w.normalized.as<bf16_t>();
-        fc.b = fc16;
-        fc.c = w.proj.as<bf16_t>();
-        fc.m = rows;
-        fc.n = fc.k = fc.lda = fc.ldb = fc.ldc = H;
-        fc.partial = w.partial.as<float>();
-        fc.partial_floats = kPrefillPartialFloats;
-        fc.epilogue = kGemmScaleBiasSilu;
-        fc.scales = m_.text_fc1_.scales;
-        fc.bias = m_.text_fc1_bias_;
-        check_hip(launch_gemm_dma(fc, stream_), "prompt text fc1");
-        fc.a = w.proj.as<bf16_t>();
-        fc.b = fc16 + static_cast<size_t>(H) * H;
-        fc.c = hidden;
-        fc.epilogue = kGemmScaleBias;
-        fc.scales = m_.text_fc2_.scales;
-        fc.bias = m_.text_fc2_bias_;
-        check_hip(launch_gemm_dma(fc, stream_), "prompt text fc2");
-        check_hip(launch_prompt_rows(hidden, text_ids, codec_ids, m_.codec_embedding_, cfg_.talker_vocab, rows, H, stream_),
-                  "prompt rows");
-        auto gemm = [&](const bf16_t* a, int lda, const bf16_t* weight, bf16_t* c, int ldc, int n, int k,
-                        const char* what, int epilogue = kGemmStore) {
+        auto gemm = [&](const bf16_t* a, int lda, const bf16_t* weight, bf16_t* c, int ldc, int n, int k) {
             Bf16GemmArgs g;
-            g.epilogue = epilogue;
             g.a = a;
             g.b = weight;
             g.c = c;
@@ -779,8 +742,29 @@ public:
             g.ldc = ldc;
             g.partial = w.partial.as<float>();
             g.partial_floats = kPrefillPartialFloats;
-            check_hip(launch_bf16_gemm(g, stream_), what);
+            return g;
         };
+        // prompt embeddings: int8 text projection, then zero text-less rows
+        // and add codec embeddings.  The integers run as bf16 (exactly) on the
+        // matrix cores, scale and bias in the epilogue: the same products
+        // summed in fp32, in another order than the decode step's GEMVs
+        // (512 rows: 318 us as exact-order GEMVs, 35 us here).
+        check_hip(launch_gather_text_rows(m_.text_embedding_, text_ids, cfg_.text_vocab, rows, H, w.normalized.as<bf16_t>(),
+                                          stream_),
+                  "gather prompt text embeddings");
+        const bf16_t* fc16 = m_.text16_.as<bf16_t>();
+        Bf16GemmArgs fc = gemm(w.normalized.as<bf16_t>(), H, fc16, w.proj.as<bf16_t>(), H, H, H);
+        fc.epilogue = kGemmScaleBiasSilu;
+        fc.scales = m_.text_fc1_.scales;
+        fc.bias = m_.text_fc1_bias_;
+        check_hip(launch_gemm_dma(fc, stream_), "prompt text fc1");
+        fc = gemm(w.proj.as<bf16_t>(), H, fc16 + static_cast<size_t>(H) * H, hidden, H, H, H);
+        fc.epilogue = kGemmScaleBias;
+        fc.scales = m_.text_fc2_.scales;
+        fc.bias = m_.text_fc2_bias_;
+        check_hip(launch_gemm_dma(fc, stream_), "prompt text fc2");
+        check_hip(launch_prompt_rows(hidden, text_ids, codec_ids, m_.codec_embedding_, cfg_.talker_vocab, rows, H, stream_),
+                  "prompt rows");
         bf16_t* xn = w.normalized.as<bf16_t>();
         bf16_t* qkv = w.qkv.as<bf16_t>();
         bf16_t* attn = w.attn.as<bf16_t>();
@@ -791,100 +775,31 @@ public:
             bf16_t* kc = host_bases_[l];
             bf16_t* vc = host_bases_[T.layers + l];
             check_hip(launch_rms_norm_rows(hidden, L.input_norm, xn, rows, H, cfg_.eps, stream_), "prefill input norm");
-            {  // q, k and v: one GEMM over the three weights as row segments of B
-                Bf16GemmArgs g;
-                g.a = xn;
-                g.b = L.q16;
-                g.b2 = L.k16;
-                g.b2_row = qw;
-                g.b3 = L.v16;
-                g.b3_row = qw + kvw;
-                g.c = qkv;
-                g.m = rows;
-                g.n = qkvw;
-                g.k = H;
-                g.lda = H;
-                g.ldb = H;
-                g.ldc = qkvw;
-                g.partial = w.partial.as<float>();
-                g.partial_floats = kPrefillPartialFloats;
-                check_hip(launch_bf16_gemm(g, stream_), "prefill q/k/v GEMM");
-            }
+            // q, k and v: one GEMM over the three weights as row segments of B
+            Bf16GemmArgs g = gemm(xn, H, L.q16, qkv, qkvw, qkvw, H);
+            g.b2 = L.k16;
+            g.b2_row = qw;
+            g.b3 = L.v16;
+            g.b3_row = qw + kvw;
+            check_hip(launch_bf16_gemm(g, stream_), "prefill q/k/v GEMM");
             check_hip(launch_prefill_qkv_epilogue(qkv, L.q_norm, L.k_norm, m_.rope_table_.as<bf16_t>(), kc, vc, vstride, 0,
                                                   rows, T.query_heads, T.key_value_heads, cfg_.eps, stream_),
                       "prefill q/k norm + RoPE + cache");
-            if (gemm_attention) {
-                bf16_t* scores = w.scores.as<bf16_t>();
-                bf16_t* vt = w.values_t.as<bf16_t>();
-                Bf16GemmArgs s;  // scores[h] = q_h k_h^T
-                s.a = qkv;
-                s.lda = qkvw;
-                s.a_batch = hd;
-                s.b = qkv + qw;
-                s.ldb = qkvw;
-                s.b_batch = hd;
-                s.b_group = T.query_heads / T.key_value_heads;
-                s.c = scores;
-                s.ldc = rp;
-                s.c_batch = static_cast<long long>(rows) * rp;
-                s.m = rows;
-                s.n = rows;
-                s.k = hd;
-                s.batch = T.query_heads;
-                s.partial = w.partial.as<float>();
-                s.partial_floats = kPrefillPartialFloats;
-                check_hip(launch_bf16_gemm(s, stream_), "prefill score GEMM");
-                check_hip(launch_causal_softmax(scores, T.query_heads, rows, rp, hd, stream_), "prefill causal softmax");
-                check_hip(launch_transpose_values(qkv, qkvw, qw + kvw, rows, rp, T.key_value_heads, vt, stream_),
-                          "prefill value transpose");
-                Bf16GemmArgs o;  // out_h = p_h v_h
-                o.a = scores;
-                o.lda = rp;
-                o.a_batch = static_cast<long long>(rows) * rp;
-                o.b = vt;
-                o.ldb = rp;
-                o.b_batch = static_cast<long long>(hd) * rp;
-                o.b_group = T.query_heads / T.key_value_heads;
-                o.c = attn;
-                o.ldc = qw;
-                o.c_batch = hd;
-                o.m = rows;
-                o.n = hd;
-                o.k = rp;
-                o.batch = T.query_heads;
-                o.partial = w.partial.as<float>();
-                o.partial_floats = kPrefillPartialFloats;
-                check_hip(launch_bf16_gemm(o, stream_), "prefill value GEMM");
-            } else {
-                // the exact kernel, row r over positions 0..r, in chunks that
-                // bound the score workspace
-                for (int r0 = 0; r0 < rows; r0 += kPrefillChunk) {
-                    const int n = std::min(kPrefillChunk, rows - r0);
-                    check_hip(launch_attention(true, qkv + static_cast<size_t>(r0) * qkvw, qkvw, nullptr, nullptr, kc, vc,
-                                               w.positions.as<int>() + r0, 0, attn + static_cast<size_t>(r0) * qw, n,
-                                               T.query_heads, T.key_value_heads, hd, max_seq_, w.workspace.as<float>(),
-                                               nullptr, stream_),
-                              "prefill exact attention");
-                }
-            }
+            check_hip(launch_prefill_attention(qkv, qkvw, kc, vc, vstride, attn, rows, T.query_heads, T.key_value_heads, hd,
+                                               stream_),
+                      "prefill attention");
             // O GEMM with the residual add (add_in_place) as its epilogue
-            gemm(attn, qw, L.o16, hidden, H, H, qw, "prefill O GEMM + residual", kGemmAddInto);
+            g = gemm(attn, qw, L.o16, hidden, H, H, qw);
+            g.epilogue = kGemmAddInto;
+            check_hip(launch_bf16_gemm(g, stream_), "prefill O GEMM + residual");
             check_hip(launch_rms_norm_rows(hidden, L.post_norm, xn, rows, H, cfg_.eps, stream_), "prefill post norm");
-            {  // gate and up GEMMs in one launch, silu_gate as their epilogue
-                Bf16GemmArgs g;
-                g.a = xn;
-                g.b = L.gate16;
-                g.b2 = L.up16;
-                g.c = gate;
-                g.m = rows;
-                g.n = I;
-                g.k = H;
-                g.lda = H;
-                g.ldb = H;
-                g.ldc = I;
-                check_hip(launch_gate_up_gemm(g, stream_), "prefill gate/up GEMM + SiLU gate");
-            }
-            gemm(gate, I, L.down16, hidden, H, H, I, "prefill down GEMM + residual", kGemmAddInto);
+            // gate and up GEMMs in one launch, silu_gate as their epilogue
+            g = gemm(xn, H, L.gate16, gate, I, I, H);
+            g.b2 = L.up16;
+            check_hip(launch_gate_up_gemm(g, stream_), "prefill gate/up GEMM + SiLU gate");
+            g = gemm(gate, I, L.down16, hidden, H, H, I);
+            g.epilogue = kGemmAddInto;
+            check_hip(launch_bf16_gemm(g, stream_), "prefill down GEMM + residual");
         }
     }
 
@@ -1127,13 +1042,12 @@ private:
     }
 
     // Row buffers of the bf16 prefill, grown on demand and kept.
-    static constexpr int kPrefillChunk = 128;  // rows per exact-attention launch
-    // split-K partial sums of the prefill GEMMs (short prompts), 16 MB
+    // split-K partial sums of the prefill GEMMs, 16 MB
     static constexpr size_t kPrefillPartialFloats = size_t{4} << 20;
     struct PrefillBuffers {
-        DeviceBuffer hidden, normalized, qkv, attn, proj, gate, scores, values_t, positions, workspace, partial;
-        int rows = 0, score_stride = 0, capacity = 0;
-        void ensure(int r, int H, int I, int qkvw, int qw, int query_heads, int kv_heads, int rp, int exact_capacity) {
+        DeviceBuffer hidden, normalized, qkv, attn, proj, gate, partial;
+        int rows = 0;
+        void ensure(int r, int H, int I, int qkvw, int qw) {
             const size_t b = sizeof(bf16_t);
             if (partial.as<void>() == nullptr) partial = DeviceBuffer(kPrefillPartialFloats * sizeof(float));
             if (r > rows) {
@@ -1144,20 +1058,6 @@ private:
                 proj = DeviceBuffer(static_cast<size_t>(r) * H * b);
                 gate = DeviceBuffer(static_cast<size_t>(r) * I * b);
                 rows = r;
-            }
-            if (rp > score_stride) {  // GEMM attention: scores, transposed values
-                scores = DeviceBuffer(static_cast<size_t>(query_heads) * rp * rp * b);
-                values_t = DeviceBuffer(static_cast<size_t>(kv_heads) * 128 * rp * b);
-                score_stride = rp;
-            }
-            if (exact_capacity > capacity) {  // exact attention: positions, score workspace
-                std::vector<int> ids(static_cast<size_t>(exact_capacity));
-                for (int i = 0; i < exact_capacity; ++i) ids[i] = i;
-                positions = DeviceBuffer(ids.size() * sizeof(int));
-                check_hip(hipMemcpy(positions.as<void>(), ids.data(), ids.size() * sizeof(int), hipMemcpyHostToDevice),
-                          "upload prefill positions");
-                workspace = DeviceBuffer(attention_workspace_bytes(kPrefillChunk, query_heads, exact_capacity));
-                capacity = exact_capacity;
             }
         }
     };
