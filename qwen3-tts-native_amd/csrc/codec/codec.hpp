@@ -35,24 +35,32 @@ constexpr int kStageOut[4] = {768, 384, 192, 96};
 constexpr int kStride[4] = {8, 5, 4, 3};
 constexpr int kDilation[3] = {1, 3, 9};
 
-// ---- fp32 MFMA convolution GEMM -------------------------------------------
+// ---- products (conv_gemm.hip) -----------------------------------------------
 // out[p][col] = epilogue( sum_k A[p][k] * W[col][k] ),  k = t * C + c,
 // A[p][t * C + c] = a[(p + t * dilation) * C + c].
-enum GemmEpilogue : int {
+enum ConvEpilogue : int {
     kEpStore = 0,          // v = acc + bias
     kEpGelu = 1,           // v = gelu(acc + bias)          (erf form)
     kEpGammaResidual = 2,  // v = residual + (acc + bias) * gamma
     kEpResidual = 3,       // v = (acc + bias) + residual
 };
 
-struct ConvGemmArgs {
+// Streams of a batch that share a launch.  Every session's arena has the same
+// layout: stream s's buffers lie delta[s] bytes from the first stream's, which
+// the launches' pointers name (delta[0] = 0).
+constexpr int kMaxStreams = 6;
+struct Streams {
+    int count = 1;
+    long long delta[kMaxStreams] = {};
+};
+
+struct ConvArgs {
     const float* a;
-    int channels_in;  // C: floats per extended row
-    int taps;
+    int channels_in;  // C: floats per buffer row
     int dilation;
     const float* w;  // [n][k]
     const float* bias;
-    int m, n, k;
+    int m, n, k;       // rows of one stream, columns, taps * C
     int channels_out;  // parameter index of column col is col % channels_out
     int epilogue;
     const float* residual;  // same [m][n] indexing as out
@@ -63,25 +71,11 @@ struct ConvGemmArgs {
     float* snake_out;
     const float* snake_alpha;
     const float* snake_beta_den;
-    // split-K over `splits` slices: partial sums in `partial`, reduced by a
-    // second launch
-    int splits;
-    float* partial;
+    float* partial;  // K slices' sums, [slice][rows of all streams][n]: conv_partial_floats
+    Streams streams;
 };
-
-// block tiles (rows x columns): 16x64 for 1..16 rows (weight streaming),
-// 32x32, 32x64 and 64x64 for longer sequences
-enum class GemmShape : int { k16x64 = 0, k32x32 = 1, k32x64 = 2, k64x64 = 3 };
-
-struct GemmPlan {
-    GemmShape shape;
-    int tiles_m, tiles_n, splits;
-    int k_step;  // 32 or 64 floats of K per pipeline step
-    size_t partial_floats() const;
-    size_t tiles() const { return (size_t)tiles_m * tiles_n; }
-};
-GemmPlan plan_conv_gemm(int m, int n, int k, int channels_in, int cus);
-hipError_t launch_conv_gemm(const ConvGemmArgs& args, const GemmPlan& plan, hipStream_t stream);
+hipError_t launch_conv(const ConvArgs& args, hipStream_t stream);
+size_t conv_partial_floats(int m, int n, int k, int streams);
 
 // ---- rows GEMV (1..4 rows) -------------------------------------------------
 enum RowsEpilogue : int {
@@ -104,16 +98,19 @@ struct RowsGemvArgs {
     int ldo;
     unsigned long long* advance_position;  // if set: *p += advance_by after the launch's reads
     int advance_by;
+    Streams streams;
 };
 hipError_t launch_rows_gemv(const RowsGemvArgs& args, hipStream_t stream);
 
 // ---- transformer attention --------------------------------------------------
-// RoPE (base 10000, rotate-half pairs d, d + 32) on q and k of `frames` rows of
+// RoPE (base 10000, rotate-half pairs d, d + 32; angles from `rotations`
+// [frame][32][cos, sin], written by the frontend) on q and k of `frames` rows of
 // qkv [frames][3072] at positions *position + f, appends k and v to the layer's
 // ring ([16][kKvSlots][64] each), and writes the 72-window causal attention of
 // each frame to out [frames][1024].
-hipError_t launch_codec_attention(const float* qkv, int frames, const unsigned long long* position, float* kv_k,
-                                  float* kv_v, float* out, hipStream_t stream);
+hipError_t launch_codec_attention(const float* qkv, int frames, const unsigned long long* position,
+                                  const float* rotations, float* kv_k, float* kv_v, float* out, const Streams& streams,
+                                  hipStream_t stream);
 
 // ---- frontend -----------------------------------------------------------------
 // Codebook gather: x[f][0:256] = first codebook entry, x[f][256:512] = sum of
@@ -124,18 +121,26 @@ struct CopySegment {
     float* dst;
     unsigned floats;
 };
+// Stream s's codes at codes + s * 64 (kMaxFrames * kCodebooks), not at a
+// delta.  Also the packet's RoPE cosines and sines.
 hipError_t launch_codec_frontend(const uint16_t* codes, int frames, const float* const* embeddings,
-                                 const float* const* usages, float* x, const CopySegment* seg, int segments,
+                                 const float* const* usages, float* x, const unsigned long long* position,
+                                 float* rotations, const CopySegment* seg, int segments, const Streams& streams,
                                  hipStream_t stream);
-hipError_t launch_copy_segments(const CopySegment* seg, int segments, hipStream_t stream);
+hipError_t launch_copy_segments(const CopySegment* seg, int segments, const Streams& streams, hipStream_t stream);
 
 // ---- ConvNeXt depthwise convolution (k = 7) + LayerNorm (eps 1e-6) -----------
 hipError_t launch_dwconv_layernorm(const float* ext, int positions, const float* w, const float* b,
-                                   const float* ln_w, const float* ln_b, float* out, hipStream_t stream);
+                                   const float* ln_w, const float* ln_b, float* out, const Streams& streams,
+                                   hipStream_t stream);
 
 // ---- final convolution 96 -> 1 (k = 7), clamp, 16-bit PCM --------------------
-hipError_t launch_final_conv_pcm(const float* ext, int positions, const float* w, const float* b, int16_t* pcm,
-                                 float* preclamp, float* clamped, hipStream_t stream);
+// pcm[s]: stream s's destination (device or mapped host memory)
+struct PcmTargets {
+    int16_t* pcm[kMaxStreams];
+};
+hipError_t launch_final_conv_pcm(const float* ext, int positions, const float* w, const float* b, const PcmTargets& pcm,
+                                 float* preclamp, float* clamped, const Streams& streams, hipStream_t stream);
 
 // ---- the reference's weight-free state-machine fixture (22 ints of state) -----
 hipError_t launch_fixture_packet(const uint16_t* codes, int frames, int* state, int16_t* pcm, hipStream_t stream);

@@ -2,12 +2,11 @@
 // native/qwen3-tts-native-codec/native/src/codec_state.cu, cited CS:line).
 //
 // The reference runs cuBLAS SGEMM plus one elementwise kernel per operation.
-// Here the convolutions are one fp32 MFMA GEMM kernel whose A operand is read
-// straight from the extended (history + packet) buffer -- no im2col copy --
-// and whose epilogue applies bias, GELU, ConvNeXt's gamma residual or the
-// residual-unit add, and the following SnakeBeta, writing the next layer's
-// input directly.  The transformer's 1..4-row products are a GEMV kernel with
-// RMSNorm fused on its input.
+// Here the convolutions are fp32 matrix-core kernels (conv_gemm.hip) that read
+// their input in place and whose epilogue applies bias, GELU, the residual and
+// the following SnakeBeta, writing the next layer's input directly.  This file
+// holds the transformer's 1..4-row products (RMSNorm fused) and the rest; blockIdx.z (or .y) is the stream where
+// a batch shares a launch.
 #include "codec.hpp"
 
 #include "../q3_math.h"
@@ -17,8 +16,6 @@
 namespace q3c {
 
 namespace {
-
-typedef float floatx4 __attribute__((ext_vector_type(4)));
 
 __device__ __forceinline__ float wave_sum(float v) {
     for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
@@ -37,257 +34,34 @@ inline unsigned blocks_for(size_t count, unsigned threads = 256) {
     return (unsigned)std::min<size_t>(std::max<size_t>(b, 1), 65535u * 16);
 }
 
-// ---------------------------------------------------------------------------
-// Epilogue of one output element (CS:407-412 bias, CS:860-866 GELU,
-// CS:1115-1124 residual add, ConvNeXt gamma CS:1432-1667, SnakeBeta CS:882-898)
-// ---------------------------------------------------------------------------
-__device__ __forceinline__ void conv_epilogue(const ConvGemmArgs& g, int p, int col, int ch, float acc) {
-    float v = g.bias ? acc + g.bias[ch] : acc;
-    const size_t idx = (size_t)p * g.n + col;
-    if (g.epilogue == kEpGelu) {
-        v = 0.5f * v * (1.0f + erff(v * 0.7071067811865475f));
-    } else if (g.epilogue == kEpGammaResidual) {
-        v = g.residual[idx] + v * g.gamma[ch];
-    } else if (g.epilogue == kEpResidual) {
-        v = v + g.residual[idx];
-    }
-    if (g.out) g.out[idx] = v;
-    if (g.snake_out) {
-        const float s = sinf(v * g.snake_alpha[ch]);
-        g.snake_out[idx] = v + (s * s) / g.snake_beta_den[ch];
-    }
-}
-
-// ---------------------------------------------------------------------------
-// fp32 MFMA convolution GEMM.
-//
-// 256 threads = 4 waves in a WM x WN grid; each wave owns TM x TN tiles of
-// 16 x 16 (v_mfma_f32_16x16x4_f32).  K advances 32 floats per step through
-// two LDS buffers: the block's threads read the next step's A rows (from the
-// extended buffer, at the tap's row offset) and W rows from global memory into
-// registers -- 128 contiguous bytes per row, 8 threads per row -- while the
-// waves run the current step's MFMAs from LDS, then store them into the other
-// buffer; one barrier per step.  In a step, lane (row = lane & 15,
-// group = lane >> 4) reads 8 consecutive floats at k = 8 * group of its A row
-// and of its W row, and MFMA e (0..7) takes element e, so one MFMA's four
-// k-slots are 8g + e for g = 0..3: the same k for A and W, a valid
-// (reordered) dot product.  Rows are padded to 36 floats in LDS.
-//
-// Split-K: slice z of Z covers a contiguous range of the steps and stores its
-// partial tile; conv_gemm_reduce_kernel then sums them.  (An in-kernel
-// last-arriver fix-up needs device-scope release/acquire fences, which write
-// back and invalidate L2 and cost ~100 us per launch here.)
-// ---------------------------------------------------------------------------
-template <int TM, int TN>
-__device__ __forceinline__ float* partial_slot(const ConvGemmArgs& g, size_t tiles, size_t tile, int z, int wave, int i,
-                                               int j, int lane) {
-    return g.partial + ((((size_t)z * tiles + tile) * 4 + wave) * (TM * TN) + (i * TN + j)) * 256 + lane * 4;
-}
-
-// Lane (row16 = lane & 15, group = lane >> 4) of wave `wave` holds, for its
-// 16 x 16 sub-tile (i, j), rows 4 * group + r (r = 0..3) of column row16.
-template <int TM, int TN, int WM, int WN>
-__device__ __forceinline__ void subtile_epilogue(const ConvGemmArgs& g, const floatx4& acc, int tile_m, int tile_n,
-                                                 int wave, int i, int j, int lane) {
-    constexpr int BM = 16 * TM * WM, BN = 16 * TN * WN;
-    const int wm = wave / WN, wn = wave % WN;
-    const int col0 = tile_n * BN + (wn * TN + j) * 16;
-    if (col0 >= g.n) return;  // wave-uniform (n % 16 == 0)
-    const int col = col0 + (lane & 15);
-    const int ch = col % g.channels_out;
-    const int p0 = tile_m * BM + (wm * TM + i) * 16 + 4 * (lane >> 4);
-#pragma unroll
-    for (int r = 0; r < 4; ++r)
-        if (p0 + r < g.m) conv_epilogue(g, p0 + r, col, ch, acc[r]);
-}
-
-template <int TM, int TN, int WM, int WN>
-__device__ __forceinline__ void tile_epilogue(const ConvGemmArgs& g, const floatx4 (&acc)[TM][TN], int tile_m,
-                                              int tile_n, int wave, int lane) {
-#pragma unroll
-    for (int j = 0; j < TN; ++j)
-#pragma unroll
-        for (int i = 0; i < TM; ++i) subtile_epilogue<TM, TN, WM, WN>(g, acc[i][j], tile_m, tile_n, wave, i, j, lane);
-}
-
-template <int TM, int TN, int WM, int WN, int BK>
-__global__ __launch_bounds__(256) void conv_gemm_kernel(ConvGemmArgs g) {
-    static_assert(WM * WN == 4, "4 waves");
-    static_assert(BK == 32 || BK == 64, "K step");
-    constexpr int BM = 16 * TM * WM, BN = 16 * TN * WN;
-    constexpr int VPR = BK / 4;      // float4 per row per step
-    constexpr int ROW = BK + 4;      // LDS row pitch (floats)
-    constexpr int A_VEC = BM * VPR, W_VEC = BN * VPR;
-    constexpr int A_PER = (A_VEC + 255) / 256, W_PER = (W_VEC + 255) / 256;
-    // every thread copies A_PER + W_PER vectors; rows past the tile (small
-    // tiles) are loaded from clamped addresses into spare LDS rows, unused
-    __shared__ float lds_a[2][A_PER * (256 / VPR) * ROW];
-    __shared__ float lds_w[2][W_PER * (256 / VPR) * ROW];
-    const int tid = threadIdx.x, lane = tid & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int wm = wave / WN, wn = wave % WN;
-    const int row16 = lane & 15, group = lane >> 4;
-
-    // global -> LDS copy assignment: vector v = tid + 256 * r covers row v / VPR, float4 v % VPR
-    const float* a_src[A_PER];
-    const float* w_src[W_PER];
-#pragma unroll
-    for (int r = 0; r < A_PER; ++r) {
-        const int v = tid + 256 * r;
-        const int p = min((int)(blockIdx.y * BM) + v / VPR, g.m - 1);
-        a_src[r] = g.a + (size_t)p * g.channels_in + (v % VPR) * 4;
-    }
-#pragma unroll
-    for (int r = 0; r < W_PER; ++r) {
-        const int v = tid + 256 * r;
-        const int col = min((int)(blockIdx.x * BN) + v / VPR, g.n - 1);
-        w_src[r] = g.w + (size_t)col * g.k + (v % VPR) * 4;
-    }
-
-    const int steps = g.k / BK;
-    const int s0 = (int)((long long)steps * blockIdx.z / g.splits);
-    const int s1 = (int)((long long)steps * (blockIdx.z + 1) / g.splits);
-    // (tap, channel) of the next step to load (channels_in % BK == 0)
-    int tap = (s0 * BK) / g.channels_in;
-    int chan = s0 * BK - tap * g.channels_in;
-    int s_load = s0;
-    const size_t tap_stride = (size_t)g.dilation * g.channels_in;
-
-    floatx4 acc[TM][TN];
-#pragma unroll
-    for (int i = 0; i < TM; ++i)
-#pragma unroll
-        for (int j = 0; j < TN; ++j) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
-
-    float4 a_reg[A_PER], w_reg[W_PER];
-    auto fetch = [&]() {
-        const size_t a_off = (size_t)tap * tap_stride + chan;
-        const size_t w_off = (size_t)s_load * BK;
-#pragma unroll
-        for (int r = 0; r < A_PER; ++r) a_reg[r] = load4(a_src[r] + a_off);
-#pragma unroll
-        for (int r = 0; r < W_PER; ++r) w_reg[r] = load4(w_src[r] + w_off);
-        ++s_load;
-        chan += BK;
-        if (chan == g.channels_in) {
-            chan = 0;
-            ++tap;
-        }
-    };
-    auto stash = [&](int buf) {
-#pragma unroll
-        for (int r = 0; r < A_PER; ++r) {
-            const int v = tid + 256 * r;
-            *reinterpret_cast<float4*>(&lds_a[buf][(v / VPR) * ROW + (v % VPR) * 4]) = a_reg[r];
-        }
-#pragma unroll
-        for (int r = 0; r < W_PER; ++r) {
-            const int v = tid + 256 * r;
-            *reinterpret_cast<float4*>(&lds_w[buf][(v / VPR) * ROW + (v % VPR) * 4]) = w_reg[r];
-        }
-    };
-    auto compute = [&](int buf) {
-#pragma unroll
-        for (int kh = 0; kh < BK / 32; ++kh) {
-            float4 av[TM][2], wv[TN][2];
-#pragma unroll
-            for (int i = 0; i < TM; ++i) {
-                const float* src = &lds_a[buf][((wm * TM + i) * 16 + row16) * ROW + kh * 32 + 8 * group];
-                av[i][0] = *reinterpret_cast<const float4*>(src);
-                av[i][1] = *reinterpret_cast<const float4*>(src + 4);
-            }
-#pragma unroll
-            for (int j = 0; j < TN; ++j) {
-                const float* src = &lds_w[buf][((wn * TN + j) * 16 + row16) * ROW + kh * 32 + 8 * group];
-                wv[j][0] = *reinterpret_cast<const float4*>(src);
-                wv[j][1] = *reinterpret_cast<const float4*>(src + 4);
-            }
-#pragma unroll
-            for (int e = 0; e < 8; ++e) {
-#pragma unroll
-                for (int i = 0; i < TM; ++i) {
-                    const float4& a4 = av[i][e >> 2];
-                    const float x = (e & 3) == 0 ? a4.x : (e & 3) == 1 ? a4.y : (e & 3) == 2 ? a4.z : a4.w;
-#pragma unroll
-                    for (int j = 0; j < TN; ++j) {
-                        const float4& w4 = wv[j][e >> 2];
-                        const float y = (e & 3) == 0 ? w4.x : (e & 3) == 1 ? w4.y : (e & 3) == 2 ? w4.z : w4.w;
-                        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(x, y, acc[i][j], 0, 0, 0);
-                    }
-                }
-            }
-        }
-    };
-    if (s0 < s1) {
-        fetch();
-        stash(0);
-        __syncthreads();
-        for (int s = s0; s < s1; ++s) {
-            const int buf = (s - s0) & 1;
-            const bool more = s + 1 < s1;
-            if (more) fetch();
-            compute(buf);
-            if (more) stash(buf ^ 1);
-            __syncthreads();
-        }
-    }
-    if (g.splits > 1) {
-        // partial tile of slice z, lane-major: the reduction kernel reads it back
-        // with the same thread mapping
-        const size_t tiles = (size_t)gridDim.x * gridDim.y;
-        const size_t tile = (size_t)blockIdx.y * gridDim.x + blockIdx.x;
-#pragma unroll
-        for (int i = 0; i < TM; ++i)
-#pragma unroll
-            for (int j = 0; j < TN; ++j)
-                *reinterpret_cast<floatx4*>(partial_slot<TM, TN>(g, tiles, tile, blockIdx.z, wave, i, j, lane)) =
-                    acc[i][j];
-        return;
-    }
-    tile_epilogue<TM, TN, WM, WN>(g, acc, blockIdx.y, blockIdx.x, wave, lane);
-}
-
-// Split-K reduction: one 64-lane block per 16 x 16 sub-tile (the lanes of the
-// wave that computed it) sums the slices' partials in slice order
-// (deterministic) and runs the epilogue.
-template <int TM, int TN, int WM, int WN>
-__global__ __launch_bounds__(64) void conv_gemm_reduce_kernel(ConvGemmArgs g) {
-    const int lane = threadIdx.x;
-    const int sub = blockIdx.z;  // (wave, i, j)
-    const int wave = sub / (TM * TN), i = (sub / TN) % TM, j = sub % TN;
-    const size_t tiles = (size_t)gridDim.x * gridDim.y;
-    const size_t tile = (size_t)blockIdx.y * gridDim.x + blockIdx.x;
-    floatx4 sum = *reinterpret_cast<const floatx4*>(partial_slot<TM, TN>(g, tiles, tile, 0, wave, i, j, lane));
-    // eight slices' loads in flight together, added in slice order
-    for (int z0 = 1; z0 < g.splits; z0 += 8) {
-        floatx4 v[8];
-#pragma unroll
-        for (int d = 0; d < 8; ++d) {
-            const int z = min(z0 + d, g.splits - 1);
-            v[d] = *reinterpret_cast<const floatx4*>(partial_slot<TM, TN>(g, tiles, tile, z, wave, i, j, lane));
-        }
-#pragma unroll
-        for (int d = 0; d < 8; ++d)
-            if (z0 + d < g.splits) sum += v[d];
-    }
-    subtile_epilogue<TM, TN, WM, WN>(g, sum, blockIdx.y, blockIdx.x, wave, i, j, lane);
+// `p` of the first stream, for stream s
+template <typename T>
+__device__ __forceinline__ T* of_stream(T* p, const Streams& st, int s) {
+    return s == 0 ? p : reinterpret_cast<T*>(reinterpret_cast<uintptr_t>(p) + st.delta[s]);
 }
 
 // ---------------------------------------------------------------------------
 // Rows GEMV for 1..4 rows (transformer projections, RVQ projection, causal
-// pre-convolution).  One wave per block computes one output channel: its
+// pre-convolution).  One wave computes one output channel of one stream
+// (blockIdx.y): its
 // lanes hold the rows in registers (float4 at k = 256 * c + 4 * lane, read
 // from L2), apply RMSNorm there when asked (CS:414-434: each wave reduces the
 // row's squares itself), stream each channel's weight row with float4 loads
 // and finish with a butterfly sum.  No LDS and no barrier: the launch's
-// latency is one weight read plus one reduction.
+// latency is one weight read plus one reduction.  Four channels a block: one
+// wave a block cost the packet about 5 us more.  Matrix-core tiles (16 rows, 4
+// used) were slower here:
+// 512 x 1024 3.3 -> 5.6 us, gate/up 5.2 -> 6.9 us.
 // ---------------------------------------------------------------------------
 constexpr int kMaxRows = 4;
 
+constexpr int kGemvWaves = 4;
+
 template <int kChunks>
-__global__ __launch_bounds__(64) void rows_gemv_kernel(RowsGemvArgs g) {
-    const int lane = threadIdx.x;
-    const int ch = blockIdx.x;
+__global__ __launch_bounds__(64 * kGemvWaves) void rows_gemv_kernel(RowsGemvArgs g) {
+    const int lane = threadIdx.x & 63;
+    const int ch = blockIdx.x * kGemvWaves + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const float* rows_x = of_stream(g.x, g.streams, blockIdx.y);
     const bool pair = g.epilogue == kRowsSiluPair;
     // the channel's weight row(s) first: the longest-latency reads
     float4 wa[kChunks], wb[kChunks];
@@ -302,7 +76,7 @@ __global__ __launch_bounds__(64) void rows_gemv_kernel(RowsGemvArgs g) {
     for (int r = 0; r < kMaxRows; ++r) {
         const int rr = min(r, g.rows - 1);
 #pragma unroll
-        for (int c = 0; c < kChunks; ++c) x[r][c] = load4(g.x + (size_t)rr * g.ldx + c * 256 + lane * 4);
+        for (int c = 0; c < kChunks; ++c) x[r][c] = load4(rows_x + (size_t)rr * g.ldx + c * 256 + lane * 4);
     }
     if (g.norm) {
         float4 nw[kChunks];
@@ -328,7 +102,8 @@ __global__ __launch_bounds__(64) void rows_gemv_kernel(RowsGemvArgs g) {
             }
         }
     }
-    if (g.advance_position && ch == 0 && lane == 0) *g.advance_position += g.advance_by;
+    if (g.advance_position && ch == 0 && lane == 0)
+        *of_stream(g.advance_position, g.streams, blockIdx.y) += g.advance_by;
 
     auto dot_rows = [&](const float4 (&wv)[kChunks], float (&acc)[kMaxRows]) {
 #pragma unroll
@@ -358,112 +133,124 @@ __global__ __launch_bounds__(64) void rows_gemv_kernel(RowsGemvArgs g) {
             v = (va / (1.0f + q3_expf(-va))) * vb;  // CS:687-698
         } else {
             v = g.bias ? va + g.bias[ch] : va;
-            if (g.epilogue == kRowsScaledResidual) v = g.residual[(size_t)r * g.ldo + ch] + v * g.scale[ch];
+            if (g.epilogue == kRowsScaledResidual) v = of_stream(g.residual, g.streams, blockIdx.y)[(size_t)r * g.ldo + ch] + v * g.scale[ch];
         }
-        g.out[(size_t)r * g.ldo + ch] = v;
+        of_stream(g.out, g.streams, blockIdx.y)[(size_t)r * g.ldo + ch] = v;
     }
 }
 
 // ---------------------------------------------------------------------------
 // Transformer attention of one packet (CS:464-494 RoPE, CS:496-566 sliding
-// attention).  One block per (head, frame).  Each block rotates the packet's
-// own keys itself (so no block reads a ring slot another block writes in the
-// same launch), takes older keys and values from the ring, and follows the
-// reference's per-head loop: scores, max, exponentials, the sequential
-// denominator and the ordered value sum.  Frame 0's block appends the
+// attention).  One block per (head, frame, stream).  Each block rotates the
+// packet's own keys itself (so no block reads a ring slot another block writes
+// in the same launch), takes older keys and values from the ring, and follows
+// the reference's per-head loop: scores, max, exponentials, denominator, the
+// per-term probabilities and the value sum.  Frame 0's block appends the
 // packet's keys and values to the ring.
+//
+// Latency-bound (16 heads x 1..4 frames): scores split each key's 64 products
+// over two lanes, the denominator is a wave's tree and the values run as four
+// partial sums over 18 positions each; cosines and sines come from the
+// frontend instead of powf, sinf and cosf here.  9 us a launch before,
+// 6.8 now (four frames).
 // ---------------------------------------------------------------------------
 __global__ __launch_bounds__(256) void codec_attention_kernel(const float* qkv, int frames,
-                                                              const unsigned long long* position, float* kv_k,
-                                                              float* kv_v, float* out) {
+                                                              const unsigned long long* position,
+                                                              const float* rotations, float* kv_k, float* kv_v,
+                                                              float* out, Streams streams) {
     __shared__ float q_s[64];
     __shared__ float k_s[kWindow][65];
-    __shared__ float v_s[kWindow][65];
+    __shared__ float v_s[kWindow][64];
     __shared__ float p_s[kWindow];
-    __shared__ float denom_s;
-    const int head = blockIdx.x, f = blockIdx.y;
+    __shared__ float part_s[4][64];
+    const int head = blockIdx.x, f = blockIdx.y, stream = blockIdx.z;
     const int tid = threadIdx.x;
-    const unsigned long long pos = *position;
+    qkv = of_stream(qkv, streams, stream);
+    rotations = of_stream(rotations, streams, stream);
+    const unsigned long long pos = *of_stream(position, streams, stream);
     const unsigned long long me = pos + (unsigned long long)f;
     const unsigned long long first = me + 1 > (unsigned long long)kWindow ? me + 1 - kWindow : 0ull;
     const int count = (int)(me - first + 1);
     const int old_rows = (int)(pos - first);  // window rows before the packet
-    float* ring_k = kv_k + (size_t)head * kKvSlots * 64;
-    float* ring_v = kv_v + (size_t)head * kKvSlots * 64;
+    float* ring_k = of_stream(kv_k, streams, stream) + (size_t)head * kKvSlots * 64;
+    float* ring_v = of_stream(kv_v, streams, stream) + (size_t)head * kKvSlots * 64;
     const int first_slot = (int)(first % kKvSlots);
+    // the packet's frames 0..f, rotate-half pairs (d, d + 32); frame 0's block
+    // also appends every frame's row to the ring
+    if (tid < 128 && (tid >> 5) < frames) {
+        const int g = tid >> 5, d = tid & 31;
+        const float* row = qkv + (size_t)g * 3 * 1024 + head * 64;
+        const float cosine = rotations[(g * 32 + d) * 2], sine = rotations[(g * 32 + d) * 2 + 1];
+        const float k1 = row[1024 + d], k2 = row[1024 + d + 32];
+        const float v1 = row[2048 + d], v2 = row[2048 + d + 32];
+        const float r1 = k1 * cosine - k2 * sine, r2 = k2 * cosine + k1 * sine;
+        if (g <= f) {
+            const int j = old_rows + g;
+            k_s[j][d] = r1;
+            k_s[j][d + 32] = r2;
+            v_s[j][d] = v1;
+            v_s[j][d + 32] = v2;
+        }
+        if (g == f) {
+            const float q1 = row[d], q2 = row[d + 32];
+            q_s[d] = q1 * cosine - q2 * sine;
+            q_s[d + 32] = q2 * cosine + q1 * sine;
+        }
+        if (f == 0) {
+            const int slot = (int)((pos + (unsigned long long)g) % kKvSlots);
+            ring_k[slot * 64 + d] = r1;
+            ring_k[slot * 64 + d + 32] = r2;
+            ring_v[slot * 64 + d] = v1;
+            ring_v[slot * 64 + d + 32] = v2;
+        }
+    }
     for (int idx = tid; idx < old_rows * 16; idx += 256) {  // float4 per thread
         const int j = idx >> 4, d = (idx & 15) * 4;
         int slot = first_slot + j;
         slot -= slot >= kKvSlots ? kKvSlots : 0;
         const float4 kk = load4(ring_k + slot * 64 + d), vv = load4(ring_v + slot * 64 + d);
         k_s[j][d] = kk.x, k_s[j][d + 1] = kk.y, k_s[j][d + 2] = kk.z, k_s[j][d + 3] = kk.w;
-        v_s[j][d] = vv.x, v_s[j][d + 1] = vv.y, v_s[j][d + 2] = vv.z, v_s[j][d + 3] = vv.w;
-    }
-    if (tid < (f + 1) * 32) {  // the packet's frames 0..f, rotate-half pairs (d, d + 32)
-        const int g = tid >> 5, d = tid & 31;
-        const float* row = qkv + (size_t)g * 3 * 1024 + head * 64;
-        const float frequency = 1.0f / powf(10000.0f, (float)(2 * d) / 64.0f);
-        const float angle = (float)(pos + (unsigned long long)g) * frequency;
-        const float sine = sinf(angle), cosine = cosf(angle);
-        const float k1 = row[1024 + d], k2 = row[1024 + d + 32];
-        const float r1 = k1 * cosine - k2 * sine, r2 = k2 * cosine + k1 * sine;
-        const float v1 = row[2048 + d], v2 = row[2048 + d + 32];
-        const int j = old_rows + g;
-        k_s[j][d] = r1;
-        k_s[j][d + 32] = r2;
-        v_s[j][d] = v1;
-        v_s[j][d + 32] = v2;
-        if (g == f) {
-            const float q1 = row[d], q2 = row[d + 32];
-            q_s[d] = q1 * cosine - q2 * sine;
-            q_s[d + 32] = q2 * cosine + q1 * sine;
-        }
-    }
-    if (f == 0 && tid < frames * 32) {  // append the packet's rows to the ring
-        const int g = tid >> 5, d = tid & 31;
-        const float* row = qkv + (size_t)g * 3 * 1024 + head * 64;
-        const float frequency = 1.0f / powf(10000.0f, (float)(2 * d) / 64.0f);
-        const float angle = (float)(pos + (unsigned long long)g) * frequency;
-        const float sine = sinf(angle), cosine = cosf(angle);
-        const float k1 = row[1024 + d], k2 = row[1024 + d + 32];
-        const int slot = (int)((pos + (unsigned long long)g) % kKvSlots);
-        ring_k[slot * 64 + d] = k1 * cosine - k2 * sine;
-        ring_k[slot * 64 + d + 32] = k2 * cosine + k1 * sine;
-        ring_v[slot * 64 + d] = row[2048 + d];
-        ring_v[slot * 64 + d + 32] = row[2048 + d + 32];
+        *reinterpret_cast<float4*>(&v_s[j][d]) = vv;
     }
     __syncthreads();
+    // key j = tid / 2: dims 32 (tid & 1) .. + 31, four chains
     float score = -3.402823466e+38f;
-    if (tid < count) {
-        float sc = 0.f;
-        for (int d = 0; d < 64; ++d) sc = fmaf(q_s[d], k_s[tid][d], sc);
-        score = sc * 0.125f;
+    {
+        const int j = min(tid >> 1, count - 1), d0 = 32 * (tid & 1);
+        float sc[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int d = 0; d < 32; d += 4)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) sc[i] = fmaf(q_s[d0 + d + i], k_s[j][d0 + d + i], sc[i]);
+        float dot = (sc[0] + sc[1]) + (sc[2] + sc[3]);
+        dot += __shfl_xor(dot, 1, 64);
+        if ((tid >> 1) < count) score = dot * 0.125f;
     }
-    // max over the window: waves, then the block
-    __shared__ float wmax[4];
-    float m = wave_max(score);
+    // keys lie in waves 0..2: max and denominator over them
+    __shared__ float wmax[4], wsum[4];
+    const float m = wave_max(score);
     if ((tid & 63) == 0) wmax[tid >> 6] = m;
     __syncthreads();
     const float maximum = fmaxf(fmaxf(wmax[0], wmax[1]), fmaxf(wmax[2], wmax[3]));
-    const float e = tid < count ? q3_expf(score - maximum) : 0.f;
-    if (tid < count) p_s[tid] = e;
+    const float e = (tid >> 1) < count ? q3_expf(score - maximum) : 0.f;
+    const float total = wave_sum((tid & 1) == 0 ? e : 0.f);
+    if ((tid & 63) == 0) wsum[tid >> 6] = total;
     __syncthreads();
-    if (tid == 0) {  // sequential, in window order
-        float denominator = 0.f;
-#pragma unroll
-        for (int j = 0; j < kWindow; ++j)
-            if (j < count) denominator += p_s[j];
-        denom_s = denominator;
-    }
+    const float denominator = (wsum[0] + wsum[1]) + (wsum[2] + wsum[3]);
+    if ((tid & 1) == 0 && (tid >> 1) < count) p_s[tid >> 1] = e / denominator;  // the reference's per-term probability
     __syncthreads();
-    if (tid < count) p_s[tid] = e / denom_s;  // the reference's per-term probability
-    __syncthreads();
-    if (tid < 64) {
+    {
+        const int d = tid & 63, quarter = tid >> 6;
+        const int j0 = quarter * (kWindow / 4), j1 = min(count, j0 + kWindow / 4);
         float result = 0.f;
-#pragma unroll 8
-        for (int j = 0; j < count; ++j) result = fmaf(p_s[j], v_s[j][tid], result);
-        out[(size_t)f * 1024 + head * 64 + tid] = result;
+#pragma unroll 6
+        for (int j = j0; j < j1; ++j) result = fmaf(p_s[j], v_s[j][d], result);
+        part_s[quarter][d] = result;
     }
+    __syncthreads();
+    if (tid < 64)
+        of_stream(out, streams, stream)[(size_t)f * 1024 + head * 64 + tid] =
+            (part_s[0][tid] + part_s[1][tid]) + (part_s[2][tid] + part_s[3][tid]);
 }
 
 // ---------------------------------------------------------------------------
@@ -474,20 +261,33 @@ struct FrontendTables {
     const float* usage[kCodebooks];
 };
 
-// Segment blockIdx.y, chunk `block` of `blocks`.
-__device__ void copy_segment_chunk(const CopySegment* seg, int block, int blocks) {
+// Segment blockIdx.y of stream blockIdx.z, chunk `block` of `blocks`.
+__device__ void copy_segment_chunk(const CopySegment* seg, const Streams& streams, int block, int blocks) {
     const CopySegment sg = seg[blockIdx.y];
     const unsigned n4 = sg.floats >> 2;
-    const float4* src = reinterpret_cast<const float4*>(sg.src);
-    float4* dst = reinterpret_cast<float4*>(sg.dst);
+    const float4* src = reinterpret_cast<const float4*>(of_stream(sg.src, streams, blockIdx.z));
+    float4* dst = reinterpret_cast<float4*>(of_stream(sg.dst, streams, blockIdx.z));
     for (unsigned i = block * 256 + threadIdx.x; i < n4; i += blocks * 256) dst[i] = src[i];
 }
 
-// blockIdx.y = segment; on segment row 0 the first `frames` blocks also
-// gather frame blockIdx.x's codebook entries (all 16 lookups issued at once).
+// blockIdx.y = segment, blockIdx.z = stream; on segment row 0 the first
+// `frames` blocks also gather frame blockIdx.x's codebook entries (all 16
+// lookups issued at once), and on row 1 they form the frame's RoPE angles.
 __global__ __launch_bounds__(256) void codec_frontend_kernel(const uint16_t* codes, int frames, FrontendTables t,
-                                                             float* x, const CopySegment* seg) {
+                                                             float* x, const unsigned long long* position,
+                                                             float* rotations, const CopySegment* seg,
+                                                             Streams streams) {
+    if (blockIdx.y == 1 && (int)blockIdx.x < frames && threadIdx.x < 32) {
+        const int f = blockIdx.x, d = threadIdx.x;
+        const unsigned long long at = *of_stream(position, streams, blockIdx.z) + (unsigned long long)f;
+        const float angle = (float)at * (1.0f / powf(10000.0f, (float)(2 * d) / 64.0f));
+        float* to = of_stream(rotations, streams, blockIdx.z) + (f * 32 + d) * 2;
+        to[0] = cosf(angle);
+        to[1] = sinf(angle);
+    }
     if (blockIdx.y == 0 && (int)blockIdx.x < frames) {
+        codes += blockIdx.z * (kMaxFrames * kCodebooks);
+        x = of_stream(x, streams, blockIdx.z);
         const int f = blockIdx.x, d = threadIdx.x;
         int code[kCodebooks];
         float usage[kCodebooks], emb[kCodebooks];
@@ -514,11 +314,11 @@ __global__ __launch_bounds__(256) void codec_frontend_kernel(const uint16_t* cod
         }
         x[f * 512 + 256 + d] = acoustic;
     }
-    copy_segment_chunk(seg, blockIdx.x, gridDim.x);
+    copy_segment_chunk(seg, streams, blockIdx.x, gridDim.x);
 }
 
-__global__ __launch_bounds__(256) void copy_segments_kernel(const CopySegment* seg) {
-    copy_segment_chunk(seg, blockIdx.x, gridDim.x);
+__global__ __launch_bounds__(256) void copy_segments_kernel(const CopySegment* seg, Streams streams) {
+    copy_segment_chunk(seg, streams, blockIdx.x, gridDim.x);
 }
 
 // ---------------------------------------------------------------------------
@@ -526,8 +326,11 @@ __global__ __launch_bounds__(256) void copy_segments_kernel(const CopySegment* s
 // one block per position, 4 channels per thread.
 // ---------------------------------------------------------------------------
 __global__ __launch_bounds__(256) void dwconv_layernorm_kernel(const float* ext, const float* w, const float* b,
-                                                               const float* ln_w, const float* ln_b, float* out) {
+                                                               const float* ln_w, const float* ln_b, float* out,
+                                                               Streams streams) {
     __shared__ float red[4];
+    ext = of_stream(ext, streams, blockIdx.y);
+    out = of_stream(out, streams, blockIdx.y);
     const int p = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     float y[4];
     float sum = 0.f;
@@ -570,9 +373,13 @@ __global__ __launch_bounds__(256) void dwconv_layernorm_kernel(const float* ext,
 // chain over 24 of the 96 channels (float4 reads), then the four partial sums
 // added in channel-group order.
 __global__ __launch_bounds__(256) void final_conv_pcm_kernel(const float* ext, int positions, const float* w,
-                                                             const float* b, int16_t* pcm, float* preclamp,
-                                                             float* clamped) {
+                                                             const float* b, PcmTargets targets, float* preclamp,
+                                                             float* clamped, Streams streams) {
     __shared__ float ws[96 * 7];
+    ext = of_stream(ext, streams, blockIdx.y);
+    preclamp = of_stream(preclamp, streams, blockIdx.y);
+    clamped = of_stream(clamped, streams, blockIdx.y);
+    int16_t* pcm = targets.pcm[blockIdx.y];
     for (int i = threadIdx.x; i < 96 * 7; i += 256) ws[i] = w[i];
     __syncthreads();
     const int lane = threadIdx.x & 63;
@@ -602,9 +409,9 @@ __global__ __launch_bounds__(256) void final_conv_pcm_kernel(const float* ext, i
                 g3 = __shfl(acc, (lane & 15) + 48, 64);
     if (group != 0 || p >= positions) return;
     const float v = ((acc + g1) + g2) + g3 + b[0];
-    if (preclamp) preclamp[p] = v;
+    preclamp[p] = v;
     const float c = fminf(1.0f, fmaxf(-1.0f, v));
-    if (clamped) clamped[p] = c;
+    clamped[p] = c;
     const float scaled = roundf(c * 32767.0f);
     pcm[p] = (int16_t)fminf(32767.0f, fmaxf(-32768.0f, scaled));
 }
@@ -713,135 +520,67 @@ __global__ void fill_f32_kernel(float* dst, size_t count, float value) {
 // launchers
 // ---------------------------------------------------------------------------
 namespace {
-constexpr int kTileRows[4] = {16, 32, 32, 64};
-constexpr int kTileCols[4] = {64, 32, 64, 64};
+bool valid(const Streams& s) { return s.count >= 1 && s.count <= kMaxStreams; }
 }  // namespace
-
-size_t GemmPlan::partial_floats() const {
-    if (splits <= 1) return 0;
-    const int s = (int)shape;
-    return (size_t)splits * tiles() * kTileRows[s] * kTileCols[s];
-}
-
-GemmPlan plan_conv_gemm(int m, int n, int k, int channels_in, int cus) {
-    // Blocks in flight hide the per-step load latency: weight-streaming shapes
-    // (<= 16 rows) take 16x64 tiles and split K to ~2 blocks per CU; longer
-    // sequences take the largest tile that still gives ~2 blocks per CU, and
-    // split K (to ~1.5 blocks per CU, each slice keeping >= 4 steps) only when
-    // the tiles alone do not cover the CUs: the partial round trip and the
-    // reduction launch cost more than they gain above that.  (Chosen from
-    // per-layer measurements on MI355X.)
-    GemmPlan plan;
-    // 64-float K steps (half the barriers) wherever the channels allow
-    plan.k_step = channels_in % 64 == 0 ? 64 : 32;
-    const long long want = 2LL * cus;
-    auto tiles_for = [&](GemmShape sh) {
-        const int s = (int)sh;
-        return (long long)((m + kTileRows[s] - 1) / kTileRows[s]) * ((n + kTileCols[s] - 1) / kTileCols[s]);
-    };
-    if (m <= 16) {
-        plan.shape = GemmShape::k16x64;
-    } else if (tiles_for(GemmShape::k64x64) >= want) {
-        plan.shape = GemmShape::k64x64;
-    } else if (tiles_for(GemmShape::k32x64) >= want && n % 64 == 0) {
-        plan.shape = GemmShape::k32x64;
-    } else {
-        plan.shape = GemmShape::k32x32;
-    }
-    const int s = (int)plan.shape;
-    plan.tiles_m = (m + kTileRows[s] - 1) / kTileRows[s];
-    plan.tiles_n = (n + kTileCols[s] - 1) / kTileCols[s];
-    const long long tiles = (long long)plan.tiles_m * plan.tiles_n;
-    long long splits = 1;
-    if (plan.shape == GemmShape::k16x64) {
-        splits = (want + tiles - 1) / tiles;
-    } else if (tiles < cus) {
-        splits = (3LL * cus / 2 + tiles - 1) / tiles;
-    }
-    splits = std::min<long long>(splits, std::max(1, (k / plan.k_step) / 4));
-    plan.splits = (int)std::max<long long>(1, splits);
-    return plan;
-}
-
-namespace {
-template <int TM, int TN, int WM, int WN>
-void launch_shape(const ConvGemmArgs& args, const GemmPlan& plan, hipStream_t stream) {
-    const dim3 grid(plan.tiles_n, plan.tiles_m, plan.splits);
-    if (plan.k_step == 64) {
-        conv_gemm_kernel<TM, TN, WM, WN, 64><<<grid, 256, 0, stream>>>(args);
-    } else {
-        conv_gemm_kernel<TM, TN, WM, WN, 32><<<grid, 256, 0, stream>>>(args);
-    }
-    if (plan.splits > 1)
-        conv_gemm_reduce_kernel<TM, TN, WM, WN>
-            <<<dim3(plan.tiles_n, plan.tiles_m, 4 * TM * TN), 64, 0, stream>>>(args);
-}
-}  // namespace
-
-hipError_t launch_conv_gemm(const ConvGemmArgs& args, const GemmPlan& plan, hipStream_t stream) {
-    if (args.k % plan.k_step || args.channels_in % plan.k_step || args.n % 16 || args.m < 1 ||
-        args.splits != plan.splits ||
-        (plan.splits > 1 && !args.partial))
-        return hipErrorInvalidValue;
-    switch (plan.shape) {
-        case GemmShape::k16x64: launch_shape<1, 1, 1, 4>(args, plan, stream); break;
-        case GemmShape::k32x32: launch_shape<1, 1, 2, 2>(args, plan, stream); break;
-        case GemmShape::k32x64: launch_shape<1, 2, 2, 2>(args, plan, stream); break;
-        case GemmShape::k64x64: launch_shape<2, 2, 2, 2>(args, plan, stream); break;
-    }
-    return hipGetLastError();
-}
 
 hipError_t launch_rows_gemv(const RowsGemvArgs& g, hipStream_t stream) {
-    if (g.rows < 1 || g.rows > kMaxRows || g.k % 256 || g.ldx % 4 || g.n < 1) return hipErrorInvalidValue;
-    // one output channel per single-wave block: >= 512 blocks for every
-    // projection of the decoder (n = 512 .. 3072)
-    const unsigned blocks = (unsigned)g.n;
+    if (g.rows < 1 || g.rows > kMaxRows || g.k % 256 || g.ldx % 4 || g.n < kGemvWaves || g.n % kGemvWaves ||
+        !valid(g.streams))
+        return hipErrorInvalidValue;
+    const dim3 grid(g.n / kGemvWaves, g.streams.count);
     switch (g.k / 256) {
-        case 2: rows_gemv_kernel<2><<<blocks, 64, 0, stream>>>(g); break;
-        case 4: rows_gemv_kernel<4><<<blocks, 64, 0, stream>>>(g); break;
-        case 6: rows_gemv_kernel<6><<<blocks, 64, 0, stream>>>(g); break;
+        case 2: rows_gemv_kernel<2><<<grid, 64 * kGemvWaves, 0, stream>>>(g); break;
+        case 4: rows_gemv_kernel<4><<<grid, 64 * kGemvWaves, 0, stream>>>(g); break;
+        case 6: rows_gemv_kernel<6><<<grid, 64 * kGemvWaves, 0, stream>>>(g); break;
         default: return hipErrorInvalidValue;
     }
     return hipGetLastError();
 }
 
-hipError_t launch_codec_attention(const float* qkv, int frames, const unsigned long long* position, float* kv_k,
-                                  float* kv_v, float* out, hipStream_t stream) {
-    if (frames < 1 || frames > kMaxFrames) return hipErrorInvalidValue;
-    codec_attention_kernel<<<dim3(kHeads, frames), 256, 0, stream>>>(qkv, frames, position, kv_k, kv_v, out);
+hipError_t launch_codec_attention(const float* qkv, int frames, const unsigned long long* position,
+                                  const float* rotations, float* kv_k, float* kv_v, float* out, const Streams& streams,
+                                  hipStream_t stream) {
+    if (frames < 1 || frames > kMaxFrames || !valid(streams)) return hipErrorInvalidValue;
+    codec_attention_kernel<<<dim3(kHeads, frames, streams.count), 256, 0, stream>>>(qkv, frames, position, rotations, kv_k,
+                                                                                   kv_v, out, streams);
     return hipGetLastError();
 }
 
 hipError_t launch_codec_frontend(const uint16_t* codes, int frames, const float* const* embeddings,
-                                 const float* const* usages, float* x, const CopySegment* seg, int segments,
+                                 const float* const* usages, float* x, const unsigned long long* position,
+                                 float* rotations, const CopySegment* seg, int segments, const Streams& streams,
                                  hipStream_t stream) {
-    if (frames < 1 || frames > kMaxFrames) return hipErrorInvalidValue;
+    if (frames < 1 || frames > kMaxFrames || segments < 2 || !valid(streams)) return hipErrorInvalidValue;
     FrontendTables t;
     for (int i = 0; i < kCodebooks; ++i) {
         t.emb[i] = embeddings[i];
         t.usage[i] = usages[i];
     }
-    if (segments < 1) return hipErrorInvalidValue;
-    codec_frontend_kernel<<<dim3(8, segments), 256, 0, stream>>>(codes, frames, t, x, seg);
+    codec_frontend_kernel<<<dim3(8, segments, streams.count), 256, 0, stream>>>(codes, frames, t, x, position, rotations,
+                                                                               seg, streams);
     return hipGetLastError();
 }
 
-hipError_t launch_copy_segments(const CopySegment* seg, int segments, hipStream_t stream) {
+hipError_t launch_copy_segments(const CopySegment* seg, int segments, const Streams& streams, hipStream_t stream) {
+    if (!valid(streams)) return hipErrorInvalidValue;
     if (segments <= 0) return hipSuccess;
-    copy_segments_kernel<<<dim3(8, segments), 256, 0, stream>>>(seg);
+    copy_segments_kernel<<<dim3(8, segments, streams.count), 256, 0, stream>>>(seg, streams);
     return hipGetLastError();
 }
 
 hipError_t launch_dwconv_layernorm(const float* ext, int positions, const float* w, const float* b,
-                                   const float* ln_w, const float* ln_b, float* out, hipStream_t stream) {
-    dwconv_layernorm_kernel<<<positions, 256, 0, stream>>>(ext, w, b, ln_w, ln_b, out);
+                                   const float* ln_w, const float* ln_b, float* out, const Streams& streams,
+                                   hipStream_t stream) {
+    if (positions < 1 || !valid(streams)) return hipErrorInvalidValue;
+    dwconv_layernorm_kernel<<<dim3(positions, streams.count), 256, 0, stream>>>(ext, w, b, ln_w, ln_b, out, streams);
     return hipGetLastError();
 }
 
-hipError_t launch_final_conv_pcm(const float* ext, int positions, const float* w, const float* b, int16_t* pcm,
-                                 float* preclamp, float* clamped, hipStream_t stream) {
-    final_conv_pcm_kernel<<<(positions + 63) / 64, 256, 0, stream>>>(ext, positions, w, b, pcm, preclamp, clamped);
+hipError_t launch_final_conv_pcm(const float* ext, int positions, const float* w, const float* b, const PcmTargets& pcm,
+                                 float* preclamp, float* clamped, const Streams& streams, hipStream_t stream) {
+    if (positions < 1 || !preclamp || !clamped || !valid(streams)) return hipErrorInvalidValue;
+    final_conv_pcm_kernel<<<dim3((positions + 63) / 64, streams.count), 256, 0, stream>>>(ext, positions, w, b, pcm,
+                                                                                         preclamp, clamped, streams);
     return hipGetLastError();
 }
 

@@ -239,10 +239,6 @@ struct Ext {  // an extended buffer and its history
     int channels = 0, history = 0;
 };
 
-struct Plans {
-    GemmPlan up_tconv[2], pw1[2], pw2[2], conv0, tconv[4], conv7[4], conv1[4];
-};
-
 struct Arena {
     char* base = nullptr;
     size_t used = 0;
@@ -268,8 +264,7 @@ struct Qwen3TtsCodecContextV1 {
     Qwen3TtsCodecModelV1* model = nullptr;
     bool counts_as_shared_session = false;
     hipStream_t stream = nullptr;
-    hipEvent_t start_event = nullptr, stop_event = nullptr, consumed_event = nullptr;
-    int cus = 256;
+    hipEvent_t start_event = nullptr, stop_event = nullptr, consumed_event = nullptr, join_event = nullptr;
 
     // host-side stream state (CS:1240-1290)
     uint64_t frame_position = 0, emitted_samples = 0, neural_frame_position = 0;
@@ -282,12 +277,14 @@ struct Qwen3TtsCodecContextV1 {
     // device arena
     void* arena = nullptr;
     size_t arena_bytes = 0, kv_bytes = 0, history_bytes = 0;
-    int16_t* host_pcm = nullptr;  // pinned [ring][7680]
+    int16_t* host_pcm = nullptr;  // pinned [ring][7680]; packets write the first slot's samples from the device
+    int16_t* mapped_pcm = nullptr;   // the same memory, device address
+    uint16_t* host_codes = nullptr;  // pinned, the packet's (a batch's) codes on their way to codes_in
     uint16_t* code_ring = nullptr;
     uint16_t* codes_in = nullptr;
     int16_t* pcm_ring = nullptr;
-    int16_t* pcm_dev = nullptr;
     unsigned long long* position = nullptr;
+    float* rotations = nullptr;  // [frame][32][cos, sin] of the packet
     int* fixture_state = nullptr;
     float *x_rvq = nullptr, *t_in = nullptr, *h = nullptr, *h2 = nullptr, *qkv = nullptr, *attn = nullptr,
           *act = nullptr, *t_out = nullptr;
@@ -297,9 +294,10 @@ struct Qwen3TtsCodecContextV1 {
     float *cur[4] = {}, *ext2[4] = {};
     float *preclamp = nullptr, *clamped = nullptr;
     float* partial = nullptr;
+    // K slices' sums of a batch that this session leads, allocated with its first batch
+    float* batch_partial = nullptr;
     CopySegment* seg_in[kMaxFrames + 1] = {};
     CopySegment* seg_out[kMaxFrames + 1] = {};
-    Plans plans[kMaxFrames + 1];
 
     hipGraphExec_t graphs[kMaxFrames + 1] = {};
     bool use_graphs = true;
@@ -322,12 +320,34 @@ int segments_for_stop(int stop) {
     }
 }
 
+// K slices' workspace: the largest over the packet's products and frame counts
+size_t partial_floats(int streams) {
+    size_t most = 0;
+    auto add = [&](int m, int n, int k) { most = std::max(most, conv_partial_floats(m, n, k, streams)); };
+    for (int f = 1; f <= kMaxFrames; ++f) {
+        for (int u = 0; u < 2; ++u) {
+            const int m = f << u;  // 1x / 2x frames in, then 2x / 4x after the transposed conv
+            add(m, 2048, 1024);
+            add(2 * m, 4096, 1024);
+            add(2 * m, 1024, 4096);
+        }
+        add(4 * f, 1536, 7 * 1024);
+        for (int t = 0; t < 4; ++t) {
+            const int p_in = (int)stage_input_positions(t, f), p_out = p_in * kStride[t];
+            add(p_in, kStride[t] * kStageOut[t], 2 * kStageIn[t]);
+            add(p_out, kStageOut[t], 7 * kStageOut[t]);
+            add(p_out, kStageOut[t], kStageOut[t]);
+        }
+    }
+    return most;
+}
+
 void layout_session(Qwen3TtsCodecContextV1* s, Arena& a) {
     s->code_ring = a.take<uint16_t>(kRingSlots * kMaxFrames * kCodebooks);
-    s->codes_in = a.take<uint16_t>(kMaxFrames * kCodebooks);
+    s->codes_in = a.take<uint16_t>(kMaxStreams * kMaxFrames * kCodebooks);  // a batch's leader holds every stream's
     s->pcm_ring = a.take<int16_t>((size_t)kRingSlots * kMaxSamples);
-    s->pcm_dev = a.take<int16_t>(kMaxSamples);
     s->position = a.take<unsigned long long>(1);
+    s->rotations = a.take<float>(kMaxFrames * 64);
     s->fixture_state = a.take<int>(22);
     const size_t kv_start = a.used;
     s->kv_k = a.take<float>((size_t)kLayers * kHeads * kKvSlots * kHeadDim);
@@ -369,32 +389,7 @@ void layout_session(Qwen3TtsCodecContextV1* s, Arena& a) {
     s->preclamp = a.take<float>((size_t)F * kSamplesPerFrame);
     s->clamped = a.take<float>((size_t)F * kSamplesPerFrame);
     s->history_bytes = hist;
-    // split-K workspace: the largest plan over every frame count
-    size_t partial = 0;
-    for (int f = 1; f <= kMaxFrames; ++f) {
-        Plans& p = s->plans[f];
-        for (int u = 0; u < 2; ++u) {
-            const int m = f << u;  // 1x / 2x frames in, then 2x / 4x after the transposed conv
-            p.up_tconv[u] = plan_conv_gemm(m, 2048, 1024, 1024, s->cus);
-            p.pw1[u] = plan_conv_gemm(2 * m, 4096, 1024, 1024, s->cus);
-            p.pw2[u] = plan_conv_gemm(2 * m, 1024, 4096, 4096, s->cus);
-        }
-        p.conv0 = plan_conv_gemm(4 * f, 1536, 7 * 1024, 1024, s->cus);
-        for (int t = 0; t < 4; ++t) {
-            const int p_in = (int)stage_input_positions(t, f), p_out = p_in * kStride[t];
-            p.tconv[t] = plan_conv_gemm(p_in, kStride[t] * kStageOut[t], 2 * kStageIn[t], kStageIn[t], s->cus);
-            p.conv7[t] = plan_conv_gemm(p_out, kStageOut[t], 7 * kStageOut[t], kStageOut[t], s->cus);
-            p.conv1[t] = plan_conv_gemm(p_out, kStageOut[t], kStageOut[t], kStageOut[t], s->cus);
-        }
-        const GemmPlan* all[] = {&p.up_tconv[0], &p.up_tconv[1], &p.pw1[0], &p.pw1[1], &p.pw2[0], &p.pw2[1],
-                                 &p.conv0, &p.tconv[0], &p.tconv[1], &p.tconv[2], &p.tconv[3], &p.conv7[0],
-                                 &p.conv7[1], &p.conv7[2], &p.conv7[3], &p.conv1[0], &p.conv1[1], &p.conv1[2],
-                                 &p.conv1[3]};
-        for (const GemmPlan* g : all) {
-            partial = std::max(partial, g->partial_floats());
-        }
-    }
-    s->partial = a.take<float>(std::max<size_t>(partial, 1));
+    s->partial = a.take<float>(std::max<size_t>(partial_floats(1), 1));
     for (int f = 0; f <= kMaxFrames; ++f) {
         s->seg_in[f] = a.take<CopySegment>(kSegments);
         s->seg_out[f] = a.take<CopySegment>(kSegments);
@@ -459,57 +454,88 @@ hipError_t reset_device_state(Qwen3TtsCodecContextV1* s) {
 // packet launch sequence (CS:3989-4089 and the stages it calls)
 // ---------------------------------------------------------------------------
 struct Launcher {
-    Qwen3TtsCodecContextV1* s;
+    Qwen3TtsCodecContextV1* s;  // the first stream
     const Weights& w;
+    Streams streams;
+    PcmTargets pcm;
+    float* partial;
     hipError_t st = hipSuccess;
+
+    explicit Launcher(Qwen3TtsCodecContextV1* one) : s(one), w(one->model->w), pcm{}, partial(one->partial) {
+        pcm.pcm[0] = one->mapped_pcm;
+    }
+    // sessions of one model, each on its own arena
+    Launcher(Qwen3TtsCodecContextV1* const* group, int count)
+        : s(group[0]), w(group[0]->model->w), pcm{}, partial(group[0]->batch_partial) {
+        streams.count = count;
+        for (int i = 0; i < count; ++i) {
+            streams.delta[i] = static_cast<char*>(group[i]->arena) - static_cast<char*>(group[0]->arena);
+            pcm.pcm[i] = group[i]->mapped_pcm;
+        }
+    }
 
     void ok(hipError_t e) {
         if (st == hipSuccess) st = e;
     }
 
     void rows(const float* x, int ldx, int rows, int k, int n, const float* wt, const float* norm, const float* bias,
-              int epilogue, const float* residual, const float* scale, float* out, int ldo,
+              int epilogue, const float* residual, const float* scale, float* out,
               unsigned long long* advance = nullptr, int by = 0) {
-        RowsGemvArgs g{x, ldx, rows, k, n, wt, norm, bias, epilogue, residual, scale, out, ldo, advance, by};
+        RowsGemvArgs g{x, ldx, rows, k, n, wt, norm, bias, epilogue, residual, scale, out, n, advance, by, streams};
         ok(launch_rows_gemv(g, s->stream));
     }
 
-    void gemm(const GemmPlan& plan, const float* a, int cin, int taps, int dilation, const float* wt,
-              const float* bias, int m, int n, int k, int cout, int epilogue, const float* residual,
-              const float* gamma, float* out, float* snake_out, const float* alpha, const float* beta) {
-        ConvGemmArgs g{a,   cin,    taps,     dilation, wt,    bias,      m,     n,     k,
-                       cout, epilogue, residual, gamma,    out,   snake_out, alpha, beta, plan.splits,
-                       s->partial};
-        ok(launch_conv_gemm(g, plan, s->stream));
+    void gemm(const float* a, int cin, int taps, int dilation, const float* wt, const float* bias, int m, int n,
+              int cout, int epilogue, const float* residual, const float* gamma, float* out, float* snake_out,
+              const float* alpha, const float* beta) {
+        ConvArgs g{};
+        g.a = a;
+        g.channels_in = cin;
+        g.dilation = dilation;
+        g.w = wt;
+        g.bias = bias;
+        g.m = m;
+        g.n = n;
+        g.k = taps * cin;
+        g.channels_out = cout;
+        g.epilogue = epilogue;
+        g.residual = residual;
+        g.gamma = gamma;
+        g.out = out;
+        g.snake_out = snake_out;
+        g.snake_alpha = alpha;
+        g.snake_beta_den = beta;
+        g.partial = partial;
+        g.streams = streams;
+        ok(launch_conv(g, s->stream));
     }
 
-    void history_out(int frames, int stop) { ok(launch_copy_segments(s->seg_out[frames], segments_for_stop(stop), s->stream)); }
+    void history_out(int frames, int stop) {
+        ok(launch_copy_segments(s->seg_out[frames], segments_for_stop(stop), streams, s->stream));
+    }
 
     // stop: 0 whole packet; 1 frontend; 2 transformer; 3 latent; 6..13 decoder checkpoint
     void packet(int F, int stop) {
-        const Plans& pl = s->plans[F];
-        ok(launch_codec_frontend(s->codes_in, F, w.emb, w.usage, s->x_rvq, s->seg_in[F], kSegments, s->stream));
+        ok(launch_codec_frontend(s->codes_in, F, w.emb, w.usage, s->x_rvq, s->position, s->rotations, s->seg_in[F],
+                                 kSegments, streams, s->stream));
         float* rvq = s->pre.ext + 2 * 512;
-        rows(s->x_rvq, 512, F, 512, 512, w.rvq_proj, nullptr, nullptr, kRowsStore, nullptr, nullptr, rvq, 512);
+        rows(s->x_rvq, 512, F, 512, 512, w.rvq_proj, nullptr, nullptr, kRowsStore, nullptr, nullptr, rvq);
         rows(s->pre.ext, 512, F, 3 * 512, 1024, w.preconv, nullptr, w.preconv_b, kRowsStore, nullptr, nullptr,
-             s->t_in, 1024);
+             s->t_in);
         if (stop == 1) return history_out(F, stop);
 
-        rows(s->t_in, 1024, F, 1024, 512, w.in_proj, nullptr, w.in_proj_b, kRowsStore, nullptr, nullptr, s->h, 512);
+        rows(s->t_in, 1024, F, 1024, 512, w.in_proj, nullptr, w.in_proj_b, kRowsStore, nullptr, nullptr, s->h);
         const size_t kv_layer = (size_t)kHeads * kKvSlots * kHeadDim;
         for (int l = 0; l < kLayers; ++l) {
             const LayerW& L = w.layer[l];
-            rows(s->h, 512, F, 512, 3072, L.qkv, L.in_norm, nullptr, kRowsStore, nullptr, nullptr, s->qkv, 3072);
-            ok(launch_codec_attention(s->qkv, F, s->position, s->kv_k + l * kv_layer, s->kv_v + l * kv_layer,
-                                      s->attn, s->stream));
-            rows(s->attn, 1024, F, 1024, 512, L.o, nullptr, nullptr, kRowsScaledResidual, s->h, L.attn_scale, s->h2,
-                 512);
-            rows(s->h2, 512, F, 512, 1024, L.gate_up, L.post_norm, nullptr, kRowsSiluPair, nullptr, nullptr, s->act,
-                 1024);
-            rows(s->act, 1024, F, 1024, 512, L.down, nullptr, nullptr, kRowsScaledResidual, s->h2, L.mlp_scale, s->h,
-                 512);
+            rows(s->h, 512, F, 512, 3072, L.qkv, L.in_norm, nullptr, kRowsStore, nullptr, nullptr, s->qkv);
+            ok(launch_codec_attention(s->qkv, F, s->position, s->rotations, s->kv_k + l * kv_layer,
+                                      s->kv_v + l * kv_layer, s->attn, streams, s->stream));
+            rows(s->attn, 1024, F, 1024, 512, L.o, nullptr, nullptr, kRowsScaledResidual, s->h, L.attn_scale, s->h2);
+            rows(s->h2, 512, F, 512, 1024, L.gate_up, L.post_norm, nullptr, kRowsSiluPair, nullptr, nullptr, s->act);
+            rows(s->act, 1024, F, 1024, 512, L.down, nullptr, nullptr, kRowsScaledResidual, s->h2, L.mlp_scale, s->h);
         }
-        rows(s->h, 512, F, 512, 1024, w.out_proj, w.norm, w.out_proj_b, kRowsStore, nullptr, nullptr, s->t_out, 1024,
+        rows(s->h, 512, F, 512, 1024, w.out_proj, w.norm, w.out_proj_b, kRowsStore, nullptr, nullptr, s->t_out,
              s->position, F);
         if (stop == 2) return history_out(F, stop);
 
@@ -519,13 +545,14 @@ struct Launcher {
             const UpW& U = w.up[u];
             const int m = F << u, p = 2 * m;
             float* dw_in = s->up_dw[u].ext + 6 * 1024;
-            gemm(pl.up_tconv[u], in, 1024, 1, 1, U.tconv, U.tconv_b, m, 2048, 1024, 1024, kEpStore, nullptr, nullptr,
+            gemm(in, 1024, 1, 1, U.tconv, U.tconv_b, m, 2048, 1024, kEpStore, nullptr, nullptr,
                  dw_in, nullptr, nullptr, nullptr);
-            ok(launch_dwconv_layernorm(s->up_dw[u].ext, p, U.dw, U.dw_b, U.ln_w, U.ln_b, s->ln, s->stream));
-            gemm(pl.pw1[u], s->ln, 1024, 1, 1, U.pw1, U.pw1_b, p, 4096, 1024, 4096, kEpGelu, nullptr, nullptr, s->pw,
+            ok(launch_dwconv_layernorm(s->up_dw[u].ext, p, U.dw, U.dw_b, U.ln_w, U.ln_b, s->ln, streams,
+                                       s->stream));
+            gemm(s->ln, 1024, 1, 1, U.pw1, U.pw1_b, p, 4096, 4096, kEpGelu, nullptr, nullptr, s->pw,
                  nullptr, nullptr, nullptr);
             float* out = u == 0 ? s->up1_out : s->conv0.ext + 6 * 1024;
-            gemm(pl.pw2[u], s->pw, 4096, 1, 1, U.pw2, U.pw2_b, p, 1024, 4096, 1024, kEpGammaResidual, dw_in, U.gamma,
+            gemm(s->pw, 4096, 1, 1, U.pw2, U.pw2_b, p, 1024, 1024, kEpGammaResidual, dw_in, U.gamma,
                  out, nullptr, nullptr, nullptr);
             in = out;
         }
@@ -533,19 +560,19 @@ struct Launcher {
 
         // waveform decoder
         const StageW& S0 = w.stage[0];
-        gemm(pl.conv0, s->conv0.ext, 1024, 7, 1, w.conv0, w.conv0_b, 4 * F, 1536, 7 * 1024, 1536, kEpStore, nullptr,
+        gemm(s->conv0.ext, 1024, 7, 1, w.conv0, w.conv0_b, 4 * F, 1536, 1536, kEpStore, nullptr,
              nullptr, s->conv0_raw, s->tconv[0].ext + 1536, S0.alpha, S0.beta);
         if (stop == 6) return history_out(F, stop);
         for (int t = 0; t < 4; ++t) {
             const StageW& S = w.stage[t];
             const int ci = kStageIn[t], co = kStageOut[t];
             const int p_in = (int)stage_input_positions(t, F), p = p_in * kStride[t];
-            gemm(pl.tconv[t], s->tconv[t].ext, ci, 2, 1, S.tconv, S.tconv_b, p_in, kStride[t] * co, 2 * ci, co,
+            gemm(s->tconv[t].ext, ci, 2, 1, S.tconv, S.tconv_b, p_in, kStride[t] * co, co,
                  kEpStore, nullptr, nullptr, s->cur[t], s->unit[t][0].ext + (size_t)6 * kDilation[0] * co,
                  S.unit[0].alpha1, S.unit[0].beta1);
             for (int u = 0; u < 3; ++u) {
                 const UnitW& R = S.unit[u];
-                gemm(pl.conv7[t], s->unit[t][u].ext, co, 7, kDilation[u], R.conv1, R.conv1_b, p, co, 7 * co, co,
+                gemm(s->unit[t][u].ext, co, 7, kDilation[u], R.conv1, R.conv1_b, p, co, co,
                      kEpStore, nullptr, nullptr, nullptr, s->ext2[t], R.alpha2, R.beta2);
                 float* next;
                 const float *alpha, *beta;
@@ -562,20 +589,20 @@ struct Launcher {
                     alpha = w.final_alpha;
                     beta = w.final_beta;
                 }
-                gemm(pl.conv1[t], s->ext2[t], co, 1, 1, R.conv2, R.conv2_b, p, co, co, co, kEpResidual, s->cur[t],
+                gemm(s->ext2[t], co, 1, 1, R.conv2, R.conv2_b, p, co, co, kEpResidual, s->cur[t],
                      nullptr, s->cur[t], next, alpha, beta);
             }
             if (stop == 7 + t) return history_out(F, stop);
         }
         if (stop == 11) return history_out(F, stop);
-        ok(launch_final_conv_pcm(s->final_conv.ext, F * kSamplesPerFrame, w.final_w, w.final_b, s->pcm_dev,
-                                 s->preclamp, s->clamped, s->stream));
+        ok(launch_final_conv_pcm(s->final_conv.ext, F * kSamplesPerFrame, w.final_w, w.final_b, pcm, s->preclamp,
+                                 s->clamped, streams, s->stream));
         history_out(F, 0);
     }
 };
 
 hipError_t enqueue_full_packet(Qwen3TtsCodecContextV1* s, int frames) {
-    Launcher l{s, s->model->w};
+    Launcher l(s);
     if (!s->use_graphs) {
         l.packet(frames, 0);
         return l.st;
@@ -778,22 +805,11 @@ bool host_codes_valid(const uint16_t* codes, uint32_t frames) {
     return true;
 }
 
-// stages codes already in the ring slot into the graph input, runs the
-// packet, queues the PCM copy and the stop event
-int32_t enqueue_staged_packet(Qwen3TtsCodecContextV1* s, uint32_t frames, uint32_t slot, char* error,
-                              size_t capacity) {
-    const uint16_t* staged = s->code_ring + (size_t)slot * kMaxFrames * kCodebooks;
-    hipError_t st = hipMemcpyAsync(s->codes_in, staged, (size_t)frames * kCodebooks * sizeof(uint16_t),
-                                   hipMemcpyDeviceToDevice, s->stream);
-    if (st == hipSuccess) st = enqueue_full_packet(s, (int)frames);
+// runs the packet whose codes are in codes_in and records its end; the PCM
+// lands in host_pcm's first slot (one packet of a session is in flight)
+int32_t enqueue_staged_packet(Qwen3TtsCodecContextV1* s, uint32_t frames, char* error, size_t capacity) {
+    hipError_t st = enqueue_full_packet(s, (int)frames);
     if (st != hipSuccess) return hip_error(error, capacity, "launch decoder packet", st);
-    const size_t samples = (size_t)frames * kSamplesPerFrame;
-    int16_t* dev_slot = s->pcm_ring + (size_t)slot * kMaxSamples;
-    st = hipMemcpyAsync(dev_slot, s->pcm_dev, samples * sizeof(int16_t), hipMemcpyDeviceToDevice, s->stream);
-    if (st != hipSuccess) return hip_error(error, capacity, "stage packet PCM", st);
-    st = hipMemcpyAsync(s->host_pcm + (size_t)slot * kMaxSamples, dev_slot, samples * sizeof(int16_t),
-                        hipMemcpyDeviceToHost, s->stream);
-    if (st != hipSuccess) return hip_error(error, capacity, "queue packet PCM copy", st);
     st = hipEventRecord(s->stop_event, s->stream);
     return st == hipSuccess ? kOk : hip_error(error, capacity, "record packet completion", st);
 }
@@ -807,7 +823,7 @@ int32_t finish_staged_packet(Qwen3TtsCodecContextV1* s, uint32_t slot, uint32_t 
     st = hipEventElapsedTime(&ms, s->start_event, s->stop_event);
     if (st != hipSuccess) return hip_error(error, capacity, "measure packet GPU time", st);
     const size_t samples = (size_t)frames * kSamplesPerFrame;
-    std::memcpy(pcm, s->host_pcm + (size_t)slot * kMaxSamples, samples * sizeof(int16_t));
+    std::memcpy(pcm, s->host_pcm, samples * sizeof(int16_t));
     const uint64_t first_frame = s->frame_position, first_sample = s->emitted_samples;
     s->frame_position += frames;
     s->emitted_samples += samples;
@@ -821,18 +837,52 @@ int32_t finish_staged_packet(Qwen3TtsCodecContextV1* s, uint32_t slot, uint32_t 
     return kOk;
 }
 
-int32_t begin_host_packet(Qwen3TtsCodecContextV1* s, const uint16_t* codes, uint32_t frames, uint32_t* slot_out,
-                          char* error, size_t capacity) {
-    const uint32_t slot = s->next_ring_slot;
+int32_t begin_host_packet(Qwen3TtsCodecContextV1* s, const uint16_t* codes, uint32_t frames, char* error,
+                          size_t capacity) {
     hipError_t st = hipSetDevice(s->device);
     if (st != hipSuccess) return hip_error(error, capacity, "select HIP device", st);
     st = hipEventRecord(s->start_event, s->stream);
     if (st != hipSuccess) return hip_error(error, capacity, "start packet timing", st);
-    st = hipMemcpyAsync(s->code_ring + (size_t)slot * kMaxFrames * kCodebooks, codes,
-                        (size_t)frames * kCodebooks * sizeof(uint16_t), hipMemcpyHostToDevice, s->stream);
+    const size_t bytes = (size_t)frames * kCodebooks * sizeof(uint16_t);
+    std::memcpy(s->host_codes, codes, bytes);
+    st = hipMemcpyAsync(s->codes_in, s->host_codes, bytes, hipMemcpyHostToDevice, s->stream);
     if (st != hipSuccess) return hip_error(error, capacity, "upload frontend codes", st);
-    *slot_out = slot;
-    return enqueue_staged_packet(s, frames, slot, error, capacity);
+    return enqueue_staged_packet(s, frames, error, capacity);
+}
+
+// One packet of `frames` frames for each of `count` sessions of one model, as
+// one sequence of launches on the first session's stream: the weights are
+// read once and the rows of all streams fill the tiles.
+int32_t begin_host_group(Qwen3TtsCodecContextV1* const* group, const uint16_t* const* codes, int count, uint32_t frames,
+                         char* error, size_t capacity) {
+    Qwen3TtsCodecContextV1* lead = group[0];
+    hipError_t st = hipSetDevice(lead->device);
+    if (st != hipSuccess) return hip_error(error, capacity, "select HIP device", st);
+    if (!lead->batch_partial &&
+        hipMalloc(reinterpret_cast<void**>(&lead->batch_partial),
+                  std::max<size_t>(partial_floats(kMaxStreams), 1) * sizeof(float)) != hipSuccess) {
+        lead->batch_partial = nullptr;
+        write_error(error, capacity, "allocate decoder batch workspace");
+        return kAlloc;
+    }
+    // whatever the other sessions' streams still hold comes first
+    for (int i = 1; i < count && st == hipSuccess; ++i) {
+        st = hipEventRecord(group[i]->join_event, group[i]->stream);
+        if (st == hipSuccess) st = hipStreamWaitEvent(lead->stream, group[i]->join_event, 0);
+    }
+    for (int i = 0; i < count && st == hipSuccess; ++i) st = hipEventRecord(group[i]->start_event, lead->stream);
+    if (st != hipSuccess) return hip_error(error, capacity, "start packet timing", st);
+    constexpr size_t kCodes = kMaxFrames * kCodebooks;
+    for (int i = 0; i < count; ++i)
+        std::memcpy(lead->host_codes + i * kCodes, codes[i], (size_t)frames * kCodebooks * sizeof(uint16_t));
+    st = hipMemcpyAsync(lead->codes_in, lead->host_codes, count * kCodes * sizeof(uint16_t), hipMemcpyHostToDevice,
+                        lead->stream);
+    if (st != hipSuccess) return hip_error(error, capacity, "upload frontend codes", st);
+    Launcher l(group, count);
+    l.packet((int)frames, 0);
+    if (l.st != hipSuccess) return hip_error(error, capacity, "launch decoder packet", l.st);
+    for (int i = 0; i < count && st == hipSuccess; ++i) st = hipEventRecord(group[i]->stop_event, lead->stream);
+    return st == hipSuccess ? kOk : hip_error(error, capacity, "record packet completion", st);
 }
 
 int32_t check_packet_args(Qwen3TtsCodecContextV1* s, const uint16_t* codes, uint32_t frames, int32_t is_final,
@@ -871,10 +921,13 @@ void release_context(Qwen3TtsCodecContextV1* s) {
     for (auto& g : s->graphs)
         if (g) (void)hipGraphExecDestroy(g);
     if (s->arena) (void)hipFree(s->arena);
+    if (s->batch_partial) (void)hipFree(s->batch_partial);
     if (s->host_pcm) (void)hipHostFree(s->host_pcm);
+    if (s->host_codes) (void)hipHostFree(s->host_codes);
     if (s->start_event) (void)hipEventDestroy(s->start_event);
     if (s->stop_event) (void)hipEventDestroy(s->stop_event);
     if (s->consumed_event) (void)hipEventDestroy(s->consumed_event);
+    if (s->join_event) (void)hipEventDestroy(s->join_event);
     if (s->stream) (void)hipStreamDestroy(s->stream);
     (void)hipSetDevice(previous);
     if (s->model) {
@@ -917,13 +970,11 @@ int32_t create_context(int32_t device, Qwen3TtsCodecModelV1* model, bool shared_
     if (shared_session) model->active_sessions.fetch_add(1, std::memory_order_acq_rel);
     const char* graphs = std::getenv("QWEN3_TTS_CODEC_GRAPH");
     s->use_graphs = !(graphs && graphs[0] == '0');
-    hipDeviceProp_t prop{};
-    if (hipGetDeviceProperties(&prop, device) == hipSuccess && prop.multiProcessorCount > 0)
-        s->cus = prop.multiProcessorCount;
     st = hipStreamCreateWithFlags(&s->stream, hipStreamNonBlocking);
     if (st == hipSuccess) st = hipEventCreate(&s->start_event);
     if (st == hipSuccess) st = hipEventCreate(&s->stop_event);
     if (st == hipSuccess) st = hipEventCreateWithFlags(&s->consumed_event, hipEventDisableTiming);
+    if (st == hipSuccess) st = hipEventCreateWithFlags(&s->join_event, hipEventDisableTiming);
     if (st != hipSuccess) {
         release_context(s);
         return hip_error(error, capacity, "create decoder stream and events", st);
@@ -933,7 +984,10 @@ int32_t create_context(int32_t device, Qwen3TtsCodecModelV1* model, bool shared_
     s->arena_bytes = sizing.used;
     if (hipMalloc(&s->arena, s->arena_bytes) != hipSuccess ||
         hipHostMalloc(reinterpret_cast<void**>(&s->host_pcm), (size_t)kRingSlots * kMaxSamples * sizeof(int16_t),
-                      hipHostMallocDefault) != hipSuccess) {
+                      hipHostMallocDefault) != hipSuccess ||
+        hipHostGetDevicePointer(reinterpret_cast<void**>(&s->mapped_pcm), s->host_pcm, 0) != hipSuccess ||
+        hipHostMalloc(reinterpret_cast<void**>(&s->host_codes),
+                      (size_t)kMaxStreams * kMaxFrames * kCodebooks * sizeof(uint16_t), hipHostMallocDefault) != hipSuccess) {
         release_context(s);
         write_error(error, capacity, "allocate decoder session memory");
         return kAlloc;
@@ -986,7 +1040,7 @@ int32_t run_debug_prefix(Qwen3TtsCodecContextV1* s, const uint16_t* codes, uint3
         st = hipMemcpyAsync(s->codes_in, codes, (size_t)frames * kCodebooks * sizeof(uint16_t),
                             hipMemcpyHostToDevice, s->stream);
     if (st != hipSuccess) return hip_error(error, capacity, "upload frontend codes", st);
-    Launcher l{s, s->model->w};
+    Launcher l(s);
     l.packet((int)frames, stop);
     st = l.st;
     if (st == hipSuccess) st = hipStreamSynchronize(s->stream);
@@ -1352,10 +1406,9 @@ QWEN3_TTS_CODEC_API int32_t qwen3_tts_codec_process_packet_v1(Qwen3TtsCodecConte
                                   result, error, error_capacity);
     if (r != kOk) return r;
     const auto start = std::chrono::steady_clock::now();
-    uint32_t slot = 0;
-    r = begin_host_packet(context, codec_frames, frame_count, &slot, error, error_capacity);
+    r = begin_host_packet(context, codec_frames, frame_count, error, error_capacity);
     if (r != kOk) return r;
-    return finish_staged_packet(context, slot, frame_count, is_final, pcm_output, result, start, error,
+    return finish_staged_packet(context, context->next_ring_slot, frame_count, is_final, pcm_output, result, start, error,
                                 error_capacity);
 }
 
@@ -1403,32 +1456,58 @@ QWEN3_TTS_CODEC_API int32_t qwen3_tts_codec_process_batch_v1(Qwen3TtsCodecBatchI
             }
         }
     }
-    // Every stream's packet is queued on its own HIP stream before any is
-    // waited for, so the streams decode concurrently; items complete in
-    // order and the first failure ends the batch (earlier items are done).
+    // Items are checked in order; those before the first bad one are decoded.
+    // Packets of equal length on one model run as one sequence of launches,
+    // different groups side by side on their first session's streams, and all
+    // are queued before any is waited for.  The first failure is reported.
     // Results are cleared first: after a failed batch, an item whose packet
     // completed (and advanced its stream) is the one whose result has a
     // nonzero frame_count.
     for (uint32_t i = 0; i < item_count; ++i)
         if (items[i].result) *items[i].result = Qwen3TtsCodecPacketResultV1{};
     const auto start = std::chrono::steady_clock::now();
-    uint32_t slots[QWEN3_TTS_CODEC_MAX_BATCH_STREAMS] = {};
-    uint32_t queued = 0;
     int32_t status = kOk;
-    for (; queued < item_count; ++queued) {
-        Qwen3TtsCodecBatchItemV1& it = items[queued];
+    uint32_t checked = 0;
+    for (; checked < item_count; ++checked) {
+        const Qwen3TtsCodecBatchItemV1& it = items[checked];
         status = check_packet_args(it.context, it.codec_frames, it.frame_count, it.is_final, it.pcm_output,
                                    it.pcm_capacity_samples, it.result, error, error_capacity);
-        if (status == kOk)
-            status = begin_host_packet(it.context, it.codec_frames, it.frame_count, &slots[queued], error,
-                                       error_capacity);
         if (status != kOk) break;
     }
-    for (uint32_t i = 0; i < queued; ++i) {
-        Qwen3TtsCodecBatchItemV1& it = items[i];
+    bool queued[QWEN3_TTS_CODEC_MAX_BATCH_STREAMS] = {}, taken[QWEN3_TTS_CODEC_MAX_BATCH_STREAMS] = {};
+    static_assert(QWEN3_TTS_CODEC_MAX_BATCH_STREAMS <= kMaxStreams, "a group holds a whole batch");
+    for (uint32_t i = 0; i < checked; ++i) {
+        if (taken[i]) continue;
+        Qwen3TtsCodecContextV1* group[kMaxStreams];
+        const uint16_t* codes[kMaxStreams];
+        uint32_t index[kMaxStreams];
+        int count = 0;
+        for (uint32_t j = i; j < i + 1; ++j) {
+            if (taken[j] || items[j].context->model != items[i].context->model ||
+                items[j].frame_count != items[i].frame_count)
+                continue;
+            taken[j] = true;
+            group[count] = items[j].context;
+            codes[count] = items[j].codec_frames;
+            index[count++] = j;
+        }
         char* e = status == kOk ? error : nullptr;
-        const int32_t r = finish_staged_packet(it.context, slots[i], it.frame_count, it.is_final, it.pcm_output,
-                                               it.result, start, e, e ? error_capacity : 0);
+        const size_t room = e ? error_capacity : 0;
+        const int32_t r = count == 1 ? begin_host_packet(group[0], codes[0], items[i].frame_count, e, room)
+                                     : begin_host_group(group, codes, count, items[i].frame_count, e, room);
+        if (r == kOk) {
+            for (int k = 0; k < count; ++k) queued[index[k]] = true;
+        } else {
+            (void)hipStreamSynchronize(group[0]->stream);  // no launch of a failed group outlives the call
+            if (status == kOk) status = r;
+        }
+    }
+    for (uint32_t i = 0; i < checked; ++i) {
+        if (!queued[i]) continue;
+        const Qwen3TtsCodecBatchItemV1& it = items[i];
+        char* e = status == kOk ? error : nullptr;
+        const int32_t r = finish_staged_packet(it.context, it.context->next_ring_slot, it.frame_count, it.is_final,
+                                               it.pcm_output, it.result, start, e, e ? error_capacity : 0);
         if (status == kOk && r != kOk) status = r;
     }
     return status;
@@ -1727,11 +1806,11 @@ QWEN3_TTS_CODEC_API int32_t qwen3_tts_codec_session_process_device_packet_begin_
     }
     const auto start = std::chrono::steady_clock::now();
     const uint32_t slot = session->next_ring_slot;
-    uint16_t* staged = session->code_ring + (size_t)slot * kMaxFrames * kCodebooks;
+    // the snapshot: codes_in is read by this packet alone (one is in flight)
     st = hipStreamWaitEvent(session->stream, reinterpret_cast<hipEvent_t>(request->producer_ready_event), 0);
     if (st == hipSuccess) st = hipEventRecord(session->start_event, session->stream);
     if (st == hipSuccess)
-        st = hipMemcpyAsync(staged, request->device_codec_frames,
+        st = hipMemcpyAsync(session->codes_in, request->device_codec_frames,
                             (size_t)request->frame_count * kCodebooks * sizeof(uint16_t), hipMemcpyDeviceToDevice,
                             session->stream);
     if (st == hipSuccess) st = hipEventRecord(session->consumed_event, session->stream);
@@ -1741,7 +1820,7 @@ QWEN3_TTS_CODEC_API int32_t qwen3_tts_codec_session_process_device_packet_begin_
         session->cancelled = true;
         return failure;
     }
-    r = enqueue_staged_packet(session, request->frame_count, slot, error, error_capacity);
+    r = enqueue_staged_packet(session, request->frame_count, error, error_capacity);
     if (r != kOk) {
         (void)hipStreamSynchronize(session->stream);
         session->cancelled = true;

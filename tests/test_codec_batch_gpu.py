@@ -1,0 +1,66 @@
+"""Packets of several streams that share their launches: each stream's PCM is
+the bits it gets alone, whatever the other streams' packet sizes, and every
+packet size agrees with the float64 whole-utterance model."""
+import numpy as np
+import pytest
+
+import codec_model as M
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def codec():
+    import qwen3_tts_codec_hip
+
+    qwen3_tts_codec_hip.load()
+    return qwen3_tts_codec_hip
+
+
+@pytest.fixture(scope="module")
+def weights():
+    return M.make_weights(3)
+
+
+@pytest.fixture(scope="module")
+def model(codec, weights):
+    return codec.SharedModel(weights)
+
+
+# packet sizes per round: groups of one to six equal packets, mixed sizes, a
+# leader that changes between rounds
+@pytest.mark.parametrize("rounds", [
+    [(4, 4, 4, 4, 4, 4), (1, 1, 1, 1, 1, 1), (4, 4, 4, 4, 4, 4)],
+    [(1, 4, 1), (4, 4, 1), (2, 3, 2)],
+    [(2, 3, 2, 3, 4), (3, 3, 3, 3, 3), (1, 2, 2, 2, 2)]])
+def test_shared_launches_give_each_stream_its_own_bits(codec, model, rounds):
+    n = len(rounds[0])
+    streams = [M.random_codes(sum(r[i] for r in rounds), 50 + i) for i in range(n)]
+    batch = [model.session() for _ in range(n)]
+    alone = [model.session() for _ in range(n)]
+    at = [0] * n
+    for sizes in rounds:
+        parts = [streams[i][at[i]:at[i] + sizes[i]] for i in range(n)]
+        got = codec.process_batch(batch, parts)
+        for i in range(n):
+            want, _ = alone[i].packet(parts[i])
+            pcm, result = got[i]
+            assert result.frame_count == sizes[i] and result.first_frame_position == at[i]
+            assert np.array_equal(pcm, want), (sizes, i)
+            at[i] += sizes[i]
+    # the same sessions go on alone, in the other order
+    for i in reversed(range(n)):
+        a, _ = batch[i].packet(streams[i][:2])
+        b, _ = alone[i].packet(streams[i][:2])
+        assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("frames", [1, 2, 3, 4])
+def test_packet_size_matches_float64(model, weights, frames):
+    """Final convolution before and after the clamp, within the published bar
+    of the reference's own checkpoint (5e-6 on the final pre-clamp)."""
+    codes = M.random_codes(2 * frames, 9)
+    whole = M.F64Decoder(weights).run(codes)
+    s = model.session()
+    got = np.concatenate([s.debug_checkpoint(codes[at:at + frames], 12, 1920 * frames, 1) for at in (0, frames)])
+    assert np.abs(got - whole[12]).max() <= 5e-6 * max(1.0, np.abs(whole[12]).max())
