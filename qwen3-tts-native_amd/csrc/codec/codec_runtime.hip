@@ -1482,7 +1482,7 @@ QWEN3_TTS_CODEC_API int32_t qwen3_tts_codec_process_batch_v1(Qwen3TtsCodecBatchI
         const uint16_t* codes[kMaxStreams];
         uint32_t index[kMaxStreams];
         int count = 0;
-        for (uint32_t j = i; j < i + 1; ++j) {
+        for (uint32_t j = i; j < checked; ++j) {
             if (taken[j] || items[j].context->model != items[i].context->model ||
                 items[j].frame_count != items[i].frame_count)
                 continue;
