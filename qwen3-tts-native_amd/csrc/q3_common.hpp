@@ -478,6 +478,10 @@ struct Bf16GemmArgs {
     int b2_row = 0, b3_row = 0;
     const float* scales = nullptr;   // kGemmScaleBias*: per column
     const bf16_t* bias = nullptr;
+    // launch_gemm_dma: RMSNorm of C's finished rows into norm_out [m][n], or null
+    const bf16_t* norm_weight = nullptr;
+    bf16_t* norm_out = nullptr;
+    float norm_epsilon = 0.f;
 };
 hipError_t launch_bf16_gemm(const Bf16GemmArgs& args, hipStream_t stream);
 // The same products through direct-to-LDS loads (gemm_dma.hip): unbatched, K a

@@ -770,11 +770,12 @@ public:
         bf16_t* attn = w.attn.as<bf16_t>();
         bf16_t* gate = w.gate.as<bf16_t>();
         const int vstride = value_cache_stride(max_seq_);
+        check_hip(launch_rms_norm_rows(hidden, m_.talker_layers_[0].input_norm, xn, rows, H, cfg_.eps, stream_),
+                  "prefill input norm");
         for (int l = 0; l < T.layers; ++l) {
             const Layer& L = m_.talker_layers_[l];
             bf16_t* kc = host_bases_[l];
             bf16_t* vc = host_bases_[T.layers + l];
-            check_hip(launch_rms_norm_rows(hidden, L.input_norm, xn, rows, H, cfg_.eps, stream_), "prefill input norm");
             // q, k and v: one GEMM over the three weights as row segments of B
             Bf16GemmArgs g = gemm(xn, H, L.q16, qkv, qkvw, qkvw, H);
             g.b2 = L.k16;
@@ -788,18 +789,27 @@ public:
             check_hip(launch_prefill_attention(qkv, qkvw, kc, vc, vstride, attn, rows, T.query_heads, T.key_value_heads, hd,
                                                stream_),
                       "prefill attention");
-            // O GEMM with the residual add (add_in_place) as its epilogue
+            // O GEMM with the residual add (add_in_place) as its epilogue, and
+            // the post-attention norm
             g = gemm(attn, qw, L.o16, hidden, H, H, qw);
             g.epilogue = kGemmAddInto;
-            check_hip(launch_bf16_gemm(g, stream_), "prefill O GEMM + residual");
-            check_hip(launch_rms_norm_rows(hidden, L.post_norm, xn, rows, H, cfg_.eps, stream_), "prefill post norm");
+            g.norm_weight = L.post_norm;
+            g.norm_out = xn;
+            g.norm_epsilon = cfg_.eps;
+            check_hip(launch_gemm_dma(g, stream_), "prefill O GEMM + residual + post norm");
             // gate and up GEMMs in one launch, silu_gate as their epilogue
             g = gemm(xn, H, L.gate16, gate, I, I, H);
             g.b2 = L.up16;
             check_hip(launch_gate_up_gemm(g, stream_), "prefill gate/up GEMM + SiLU gate");
+            // down GEMM with the residual add and the next layer's input norm
             g = gemm(gate, I, L.down16, hidden, H, H, I);
             g.epilogue = kGemmAddInto;
-            check_hip(launch_bf16_gemm(g, stream_), "prefill down GEMM + residual");
+            if (l + 1 < T.layers) {
+                g.norm_weight = m_.talker_layers_[l + 1].input_norm;
+                g.norm_out = xn;
+                g.norm_epsilon = cfg_.eps;
+            }
+            check_hip(launch_gemm_dma(g, stream_), "prefill down GEMM + residual + input norm");
         }
     }
 
