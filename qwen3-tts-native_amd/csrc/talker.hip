@@ -658,25 +658,32 @@ public:
         const SamplingParams sp = params_of(sampling);
         if (history_count_ >= max_seq_) throw std::runtime_error("semantic history exceeds configured sequence capacity");
         try {
-            DeviceBuffer prompt(static_cast<size_t>(count) * 2 * sizeof(int));
-            std::vector<int> ids(static_cast<size_t>(count) * 2);
-            std::copy(text, text + count, ids.begin());
-            std::copy(codec, codec + count, ids.begin() + count);
-            check_hip(hipMemcpyAsync(prompt.as<void>(), ids.data(), ids.size() * sizeof(int), hipMemcpyHostToDevice, stream_), "upload prompt");
-            const int zeros[2] = {0, 0};
-            check_hip(hipMemcpyAsync(ints_.as<int>(), zeros, sizeof(zeros), hipMemcpyHostToDevice, stream_), "reset position");
+            // ids and counters through pinned memory (the previous prefill's
+            // copies are complete: it ended with a synchronization)
+            prompt_.ensure(count);
+            const int* prompt = prompt_.device.as<int>();
+            std::copy(text, text + count, prompt_.host);
+            std::copy(codec, codec + count, prompt_.host + count);
+            check_hip(hipMemcpyAsync(prompt_.device.as<void>(), prompt_.host, static_cast<size_t>(count) * 2 * sizeof(int),
+                                     hipMemcpyHostToDevice, stream_),
+                      "upload prompt");
+            const bool bf16 = bf16_prefill_enabled();
+            // the GEMM prefill does not read the position: it is set to the
+            // prompt's end at once; the decode step counts up to it
+            pinned_[2] = bf16 ? count : 0;
+            pinned_[3] = 0;
+            check_hip(hipMemcpyAsync(ints_.as<int>(), pinned_ + 2, 2 * sizeof(int), hipMemcpyHostToDevice, stream_), "reset position");
             position_ = 0;
             history_count_ = 0;
             check_hip(hipEventRecord(start_, stream_), "hipEventRecord(prefill start)");
             const int H = cfg_.talker.hidden;
-            const bool bf16 = bf16_prefill_enabled();
             if (bf16) {
-                prefill_bf16(count, prompt.as<int>(), prompt.as<int>() + count);
+                prefill_bf16(count, prompt, prompt + count);
                 emit_prefill_logits(count);
             }
             for (int i = 0; !bf16 && i < count; ++i) {
-                const int* text_id = prompt.as<int>() + i;
-                const int* codec_id = prompt.as<int>() + count + i;
+                const int* text_id = prompt + i;
+                const int* codec_id = prompt + count + i;
                 if (text[i] >= 0) {
                     project_text(text_id, false);
                 } else {
@@ -728,7 +735,7 @@ public:
         const int qkvw = T.qkv_width(), hd = T.head_dimension;
         PrefillBuffers& w = prefill_;
         w.ensure(rows, H, I, qkvw, qw);
-        bf16_t* hidden = w.hidden.as<bf16_t>();
+        bf16_t* hidden = w.hidden;
         auto gemm = [&](const bf16_t* a, int lda, const bf16_t* weight, bf16_t* c, int ldc, int n, int k) {
             Bf16GemmArgs g;
             g.a = a;
@@ -740,7 +747,7 @@ public:
             g.lda = lda;
             g.ldb = k;
             g.ldc = ldc;
-            g.partial = w.partial.as<float>();
+            g.partial = w.partial;
             g.partial_floats = kPrefillPartialFloats;
             return g;
         };
@@ -749,26 +756,26 @@ public:
         // matrix cores, scale and bias in the epilogue: the same products
         // summed in fp32, in another order than the decode step's GEMVs
         // (512 rows: 318 us as exact-order GEMVs, 35 us here).
-        check_hip(launch_gather_text_rows(m_.text_embedding_, text_ids, cfg_.text_vocab, rows, H, w.normalized.as<bf16_t>(),
+        check_hip(launch_gather_text_rows(m_.text_embedding_, text_ids, cfg_.text_vocab, rows, H, w.normalized,
                                           stream_),
                   "gather prompt text embeddings");
         const bf16_t* fc16 = m_.text16_.as<bf16_t>();
-        Bf16GemmArgs fc = gemm(w.normalized.as<bf16_t>(), H, fc16, w.proj.as<bf16_t>(), H, H, H);
+        Bf16GemmArgs fc = gemm(w.normalized, H, fc16, w.proj, H, H, H);
         fc.epilogue = kGemmScaleBiasSilu;
         fc.scales = m_.text_fc1_.scales;
         fc.bias = m_.text_fc1_bias_;
         check_hip(launch_gemm_dma(fc, stream_), "prompt text fc1");
-        fc = gemm(w.proj.as<bf16_t>(), H, fc16 + static_cast<size_t>(H) * H, hidden, H, H, H);
+        fc = gemm(w.proj, H, fc16 + static_cast<size_t>(H) * H, hidden, H, H, H);
         fc.epilogue = kGemmScaleBias;
         fc.scales = m_.text_fc2_.scales;
         fc.bias = m_.text_fc2_bias_;
         check_hip(launch_gemm_dma(fc, stream_), "prompt text fc2");
         check_hip(launch_prompt_rows(hidden, text_ids, codec_ids, m_.codec_embedding_, cfg_.talker_vocab, rows, H, stream_),
                   "prompt rows");
-        bf16_t* xn = w.normalized.as<bf16_t>();
-        bf16_t* qkv = w.qkv.as<bf16_t>();
-        bf16_t* attn = w.attn.as<bf16_t>();
-        bf16_t* gate = w.gate.as<bf16_t>();
+        bf16_t* xn = w.normalized;
+        bf16_t* qkv = w.qkv;
+        bf16_t* attn = w.attn;
+        bf16_t* gate = w.gate;
         const int vstride = value_cache_stride(max_seq_);
         check_hip(launch_rms_norm_rows(hidden, m_.talker_layers_[0].input_norm, xn, rows, H, cfg_.eps, stream_),
                   "prefill input norm");
@@ -814,11 +821,10 @@ public:
     }
 
     // run_talker_prefill's tail (talker.cu:3204-3231): final norm of the last
-    // row into last_hidden, bf16 codec head GEMM into the logits; position =
-    // prompt length.
+    // row into last_hidden, bf16 codec head GEMM into the logits.
     void emit_prefill_logits(int rows) {
         const int H = cfg_.talker.hidden;
-        check_hip(launch_rms_norm_rows(prefill_.hidden.as<bf16_t>() + static_cast<size_t>(rows - 1) * H, m_.talker_norm_,
+        check_hip(launch_rms_norm_rows(prefill_.hidden + static_cast<size_t>(rows - 1) * H, m_.talker_norm_,
                                        last_hidden_.as<bf16_t>(), 1, H, cfg_.eps, stream_),
                   "prefill final norm");
         Bf16GemmArgs g;
@@ -831,12 +837,9 @@ public:
         g.lda = H;
         g.ldb = H;
         g.ldc = cfg_.talker_vocab;
-        g.partial = prefill_.partial.as<float>();
+        g.partial = prefill_.partial;
         g.partial_floats = kPrefillPartialFloats;
         check_hip(launch_bf16_gemm(g, stream_), "prefill codec head GEMM");
-        pinned_[1] = rows;
-        check_hip(hipMemcpyAsync(ints_.as<int>(), &pinned_[1], sizeof(int), hipMemcpyHostToDevice, stream_),
-                  "set position");
     }
 
     // begin_frame, talker.cu:1095-1262
@@ -1054,21 +1057,50 @@ private:
     // Row buffers of the bf16 prefill, grown on demand and kept.
     // split-K partial sums of the prefill GEMMs, 16 MB
     static constexpr size_t kPrefillPartialFloats = size_t{4} << 20;
+    // One allocation: seven cost a new session's first prefill 0.8 ms.
     struct PrefillBuffers {
-        DeviceBuffer hidden, normalized, qkv, attn, proj, gate, partial;
+        DeviceBuffer arena;
+        bf16_t *hidden = nullptr, *normalized = nullptr, *qkv = nullptr, *attn = nullptr, *proj = nullptr, *gate = nullptr;
+        float* partial = nullptr;
         int rows = 0;
         void ensure(int r, int H, int I, int qkvw, int qw) {
-            const size_t b = sizeof(bf16_t);
-            if (partial.as<void>() == nullptr) partial = DeviceBuffer(kPrefillPartialFloats * sizeof(float));
-            if (r > rows) {
-                hidden = DeviceBuffer(static_cast<size_t>(r) * H * b);
-                normalized = DeviceBuffer(static_cast<size_t>(r) * H * b);
-                qkv = DeviceBuffer(static_cast<size_t>(r) * qkvw * b);
-                attn = DeviceBuffer(static_cast<size_t>(r) * qw * b);
-                proj = DeviceBuffer(static_cast<size_t>(r) * H * b);
-                gate = DeviceBuffer(static_cast<size_t>(r) * I * b);
-                rows = r;
-            }
+            if (r <= rows) return;
+            rows = 0;
+            const size_t n = static_cast<size_t>(r);
+            size_t used = kPrefillPartialFloats * sizeof(float);
+            auto take = [&](size_t elements) {
+                const size_t at = used;
+                used += (elements * sizeof(bf16_t) + 255) / 256 * 256;
+                return at;
+            };
+            const size_t at[] = {take(n * H), take(n * H), take(n * qkvw), take(n * qw), take(n * H), take(n * I)};
+            arena = DeviceBuffer(used);
+            bf16_t** const to[] = {&hidden, &normalized, &qkv, &attn, &proj, &gate};
+            for (int i = 0; i < 6; ++i) *to[i] = reinterpret_cast<bf16_t*>(arena.as<char>() + at[i]);
+            partial = arena.as<float>();
+            rows = r;
+        }
+    };
+
+    // The prompt's ids on their way to the device, grown on demand and kept: an
+    // allocation and its release cost a short prefill about 20 us.
+    struct PromptBuffers {
+        DeviceBuffer device;
+        int* host = nullptr;  // pinned
+        int capacity = 0;
+        void ensure(int count) {
+            if (count <= capacity) return;
+            device = DeviceBuffer(static_cast<size_t>(count) * 2 * sizeof(int));
+            release();
+            check_hip(hipHostMalloc(reinterpret_cast<void**>(&host), static_cast<size_t>(count) * 2 * sizeof(int),
+                                    hipHostMallocDefault),
+                      "hipHostMalloc(prompt)");
+            capacity = count;
+        }
+        void release() {
+            if (host) (void)hipHostFree(host);
+            host = nullptr;
+            capacity = 0;
         }
     };
 
@@ -1330,6 +1362,7 @@ private:
         }
         if (pinned_) (void)hipHostFree(pinned_);
         pinned_ = nullptr;
+        prompt_.release();
         for (hipEvent_t* e : {&start_, &stop_, &predictor_start_, &predictor_stop_, &codes_ready_, &semantic_ready_}) {
             if (*e) (void)hipEventDestroy(*e);
             *e = nullptr;
@@ -1355,9 +1388,10 @@ private:
     PredictorPassArgs pass_{};
     bool pred_chain_ = false;
     std::vector<bf16_t*> host_bases_;
-    int* pinned_ = nullptr;  // [0] sampled token, [1] text token, [8..] codes (u16), [20] predictor pass status
+    int* pinned_ = nullptr;  // [0] sampled token, [1] text token, [2..3] prefill counters, [8..] codes (u16), [20] predictor pass status
     Graph predictor_graph_, talker_graph_;
     PrefillBuffers prefill_;
+    PromptBuffers prompt_;
     int position_ = 0;
     int history_count_ = 0;
     uint64_t frames_ = 0, device_samples_ = 0, host_syncs_ = 0;
