@@ -22,6 +22,28 @@ __device__ __forceinline__ float wave_sum(float v) {
     return v;
 }
 
+// The wave's sums of kCount (a power of two) values: sum q in the lanes whose
+// lane / (64 / kCount) is q, added in wave_sum's pairs, so with its bits.  A
+// step halves the values a lane still carries: 7 exchanges for four sums, not
+// 24, and 10 for eight.
+template <int kCount>
+__device__ __forceinline__ float wave_sums(float (&v)[kCount]) {
+    const int lane = threadIdx.x & 63;
+    int o = 32;
+#pragma unroll
+    for (int n = kCount / 2; n > 0; n >>= 1, o >>= 1) {
+        const bool upper = lane & o;
+#pragma unroll
+        for (int i = 0; i < n; ++i) {
+            const float keep = upper ? v[i + n] : v[i], give = upper ? v[i] : v[i + n];
+            v[i] = keep + __shfl_xor(give, o, 64);
+        }
+    }
+    float sum = v[0];
+    for (; o > 0; o >>= 1) sum += __shfl_xor(sum, o, 64);
+    return sum;
+}
+
 __device__ __forceinline__ float wave_max(float v) {
     for (int o = 32; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, 64));
     return v;
@@ -47,43 +69,55 @@ __device__ __forceinline__ T* of_stream(T* p, const Streams& st, int s) {
 // lanes hold the rows in registers (float4 at k = 256 * c + 4 * lane, read
 // from L2), apply RMSNorm there when asked (CS:414-434: each wave reduces the
 // row's squares itself), stream each channel's weight row with float4 loads
-// and finish with a butterfly sum.  No LDS and no barrier: the launch's
-// latency is one weight read plus one reduction.  Four channels a block: one
-// wave a block cost the packet about 5 us more.  Matrix-core tiles (16 rows, 4
-// used) were slower here:
-// 512 x 1024 3.3 -> 5.6 us, gate/up 5.2 -> 6.9 us.
+// and finish with butterfly sums.  No LDS and no barrier: the launch's
+// latency is one weight read plus one reduction (two with the norm), so the
+// rows' sums travel together (wave_sums) and the epilogue's operands are
+// requested beside the weights (a 1-frame packet 590 -> 545 us,
+// 4 frames 757 -> 737 us, six streams 2235 -> 2189 us).  Four channels a block: one wave a block
+// cost the packet about 5 us more.  Matrix-core tiles (16 rows, 4 used) were
+// slower here: 512 x 1024 3.3 -> 5.6 us, gate/up 5.2 -> 6.9 us.
+// kRows: 1, 2 or 4, the least that holds the packet's rows.
 // ---------------------------------------------------------------------------
 constexpr int kMaxRows = 4;
 
 constexpr int kGemvWaves = 4;
 
-template <int kChunks>
+template <int kChunks, int kRows, bool kPair>
 __global__ __launch_bounds__(64 * kGemvWaves) void rows_gemv_kernel(RowsGemvArgs g) {
+    constexpr int kSums = kPair ? 2 * kRows : kRows, kLanes = 64 / kSums;
     const int lane = threadIdx.x & 63;
     const int ch = blockIdx.x * kGemvWaves + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const float* rows_x = of_stream(g.x, g.streams, blockIdx.y);
-    const bool pair = g.epilogue == kRowsSiluPair;
     // the channel's weight row(s) first: the longest-latency reads
-    float4 wa[kChunks], wb[kChunks];
+    float4 wa[kChunks], wb[kPair ? kChunks : 1];
 #pragma unroll
     for (int c = 0; c < kChunks; ++c) wa[c] = load4(g.w + (size_t)ch * g.k + c * 256 + lane * 4);
-    if (pair) {
+    if constexpr (kPair) {
 #pragma unroll
         for (int c = 0; c < kChunks; ++c) wb[c] = load4(g.w + (size_t)(g.n + ch) * g.k + c * 256 + lane * 4);
     }
-    float4 x[kMaxRows][kChunks];
+    float4 x[kRows][kChunks];
 #pragma unroll
-    for (int r = 0; r < kMaxRows; ++r) {
+    for (int r = 0; r < kRows; ++r) {
         const int rr = min(r, g.rows - 1);
 #pragma unroll
         for (int c = 0; c < kChunks; ++c) x[r][c] = load4(rows_x + (size_t)rr * g.ldx + c * 256 + lane * 4);
     }
+    // sum q (of row q) ends in the lanes from q * kLanes on, the first of
+    // which finishes it; a pair's second half follows in the upper lanes
+    const int row = lane / kLanes;
+    const size_t at = (size_t)min(row, g.rows - 1) * g.ldo + ch;
+    const bool residual_add = !kPair && g.epilogue == kRowsScaledResidual;
+    const float bias = !kPair && g.bias ? g.bias[ch] : 0.f;
+    const float scale = residual_add ? g.scale[ch] : 0.f;
+    const float residual = residual_add ? of_stream(g.residual, g.streams, blockIdx.y)[at] : 0.f;
     if (g.norm) {
         float4 nw[kChunks];
 #pragma unroll
         for (int c = 0; c < kChunks; ++c) nw[c] = load4(g.norm + c * 256 + lane * 4);
+        float square[kRows];
 #pragma unroll
-        for (int r = 0; r < kMaxRows; ++r) {
+        for (int r = 0; r < kRows; ++r) {
             float sq = 0.f;
 #pragma unroll
             for (int c = 0; c < kChunks; ++c) {
@@ -92,51 +126,51 @@ __global__ __launch_bounds__(64 * kGemvWaves) void rows_gemv_kernel(RowsGemvArgs
                 sq = fmaf(x[r][c].z, x[r][c].z, sq);
                 sq = fmaf(x[r][c].w, x[r][c].w, sq);
             }
-            const float scale = 1.0f / sqrtf(wave_sum(sq) / (float)g.k + 1.0e-5f);
+            square[r] = sq;
+        }
+        const float inverse = 1.0f / sqrtf(wave_sums(square) / (float)g.k + 1.0e-5f);
+#pragma unroll
+        for (int r = 0; r < kRows; ++r) {
+            const float by = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(inverse), r * (64 / kRows)));
 #pragma unroll
             for (int c = 0; c < kChunks; ++c) {
-                x[r][c].x = x[r][c].x * scale * nw[c].x;
-                x[r][c].y = x[r][c].y * scale * nw[c].y;
-                x[r][c].z = x[r][c].z * scale * nw[c].z;
-                x[r][c].w = x[r][c].w * scale * nw[c].w;
+                x[r][c].x = x[r][c].x * by * nw[c].x;
+                x[r][c].y = x[r][c].y * by * nw[c].y;
+                x[r][c].z = x[r][c].z * by * nw[c].z;
+                x[r][c].w = x[r][c].w * by * nw[c].w;
             }
         }
     }
     if (g.advance_position && ch == 0 && lane == 0)
         *of_stream(g.advance_position, g.streams, blockIdx.y) += g.advance_by;
 
-    auto dot_rows = [&](const float4 (&wv)[kChunks], float (&acc)[kMaxRows]) {
+    float sums[kSums];
+    auto dot_row = [&](const float4* wv, int r) {
+        float s = 0.f;
 #pragma unroll
-        for (int r = 0; r < kMaxRows; ++r) {
-            float s = 0.f;
-#pragma unroll
-            for (int c = 0; c < kChunks; ++c) {
-                s = fmaf(wv[c].x, x[r][c].x, s);
-                s = fmaf(wv[c].y, x[r][c].y, s);
-                s = fmaf(wv[c].z, x[r][c].z, s);
-                s = fmaf(wv[c].w, x[r][c].w, s);
-            }
-            acc[r] = wave_sum(s);
+        for (int c = 0; c < kChunks; ++c) {
+            s = fmaf(wv[c].x, x[r][c].x, s);
+            s = fmaf(wv[c].y, x[r][c].y, s);
+            s = fmaf(wv[c].z, x[r][c].z, s);
+            s = fmaf(wv[c].w, x[r][c].w, s);
         }
+        return s;
     };
-    float a[kMaxRows], b[kMaxRows] = {0.f, 0.f, 0.f, 0.f};
-    dot_rows(wa, a);
-    if (pair) dot_rows(wb, b);
-    const int r = lane;
-    if (r < g.rows) {
-        float va = a[0], vb = b[0];
 #pragma unroll
-        for (int q = 1; q < kMaxRows; ++q)
-            if (r == q) va = a[q], vb = b[q];
-        float v;
-        if (pair) {
-            v = (va / (1.0f + q3_expf(-va))) * vb;  // CS:687-698
-        } else {
-            v = g.bias ? va + g.bias[ch] : va;
-            if (g.epilogue == kRowsScaledResidual) v = of_stream(g.residual, g.streams, blockIdx.y)[(size_t)r * g.ldo + ch] + v * g.scale[ch];
-        }
-        of_stream(g.out, g.streams, blockIdx.y)[(size_t)r * g.ldo + ch] = v;
+    for (int r = 0; r < kRows; ++r) {
+        sums[r] = dot_row(wa, r);
+        if constexpr (kPair) sums[kRows + r] = dot_row(wb, r);
     }
+    const float va = wave_sums(sums);
+    float v;
+    if constexpr (kPair) {
+        const float vb = __shfl_xor(va, 32, 64);
+        v = (va / (1.0f + q3_expf(-va))) * vb;  // CS:687-698
+    } else {
+        v = g.bias ? va + bias : va;
+        if (residual_add) v = residual + v * scale;
+    }
+    if (lane % kLanes == 0 && row < g.rows) of_stream(g.out, g.streams, blockIdx.y)[at] = v;
 }
 
 // ---------------------------------------------------------------------------
@@ -523,15 +557,28 @@ namespace {
 bool valid(const Streams& s) { return s.count >= 1 && s.count <= kMaxStreams; }
 }  // namespace
 
+template <int kChunks, int kRows>
+static void launch_rows_count(const RowsGemvArgs& g, hipStream_t stream) {
+    const dim3 grid(g.n / kGemvWaves, g.streams.count);
+    if (g.epilogue == kRowsSiluPair) rows_gemv_kernel<kChunks, kRows, true><<<grid, 64 * kGemvWaves, 0, stream>>>(g);
+    else rows_gemv_kernel<kChunks, kRows, false><<<grid, 64 * kGemvWaves, 0, stream>>>(g);
+}
+
+template <int kChunks>
+static void launch_rows_chunks(const RowsGemvArgs& g, hipStream_t stream) {
+    if (g.rows == 1) launch_rows_count<kChunks, 1>(g, stream);
+    else if (g.rows == 2) launch_rows_count<kChunks, 2>(g, stream);
+    else launch_rows_count<kChunks, 4>(g, stream);
+}
+
 hipError_t launch_rows_gemv(const RowsGemvArgs& g, hipStream_t stream) {
     if (g.rows < 1 || g.rows > kMaxRows || g.k % 256 || g.ldx % 4 || g.n < kGemvWaves || g.n % kGemvWaves ||
         !valid(g.streams))
         return hipErrorInvalidValue;
-    const dim3 grid(g.n / kGemvWaves, g.streams.count);
     switch (g.k / 256) {
-        case 2: rows_gemv_kernel<2><<<grid, 64 * kGemvWaves, 0, stream>>>(g); break;
-        case 4: rows_gemv_kernel<4><<<grid, 64 * kGemvWaves, 0, stream>>>(g); break;
-        case 6: rows_gemv_kernel<6><<<grid, 64 * kGemvWaves, 0, stream>>>(g); break;
+        case 2: launch_rows_chunks<2>(g, stream); break;
+        case 4: launch_rows_chunks<4>(g, stream); break;
+        case 6: launch_rows_chunks<6>(g, stream); break;
         default: return hipErrorInvalidValue;
     }
     return hipGetLastError();
