@@ -372,6 +372,10 @@ hipError_t launch_tile(const Bf16GemmArgs& g, int splits, hipStream_t stream) {
     gemm_dma_kernel<kBM, kBN, kWM, kWN, kStages, kEpilogue><<<grid, 64 * kWM * kWN, 0, stream>>>(g, row_tiles, panels, per);
     hipError_t st = hipGetLastError();
     const bool norm = kEpilogue == kGemmAddInto && g.norm_out != nullptr;
+    if (kEpilogue == kGemmStore && g.open_slices != nullptr && slices > 1) {  // the consumer adds them
+        if (st == hipSuccess) *g.open_slices = slices;
+        return st;
+    }
     if constexpr (kEpilogue == kGemmAddInto) {
         if (st == hipSuccess && norm && slices > 1 && slices <= 8 && g.n <= kNormColumns) {
             gemm_dma_reduce_norm_kernel<<<g.m, 256, 0, stream>>>(g, slices);

@@ -283,11 +283,20 @@ __global__ __launch_bounds__(64) void causal_softmax_kernel(bf16_t* scores, int 
 // RoPE on q and k heads in place (the decode path's exact arithmetic and
 // RoPE table); k heads also to the key cache ([position][kv_width]), v heads
 // to the blocked dimension-major value cache.  One wave per head.
+//
+// kSliced: the projection comes as `slices` fp32 partial products, added here
+// in slice order and rounded to bf16 as their reduction would, which saves
+// that launch (bound by the launches' latency at short prompts, 33 rows 3.9 +
+// 3.0 us as two; with attention's one-head blocks, eight talker layers of
+// prefill went 684 -> 627 us at 33 rows).
+template <bool kSliced>
 __global__ __launch_bounds__(64) void prefill_qkv_epilogue_kernel(bf16_t* qkv, const bf16_t* q_norm, const bf16_t* k_norm,
                                                                   const bf16_t* rope_table, bf16_t* key_cache,
                                                                   bf16_t* value_cache, int value_stride, int first,
-                                                                  int query_heads, int key_value_heads, float epsilon) {
+                                                                  int query_heads, int key_value_heads, float epsilon,
+                                                                  const float* partial, int slices, size_t slice) {
     constexpr int kDim = 128;
+    __shared__ bf16_t head_lds[kSliced ? kDim : 1];
     const int heads = query_heads + 2 * key_value_heads;
     const int row = blockIdx.x / heads;
     const int head = blockIdx.x % heads;
@@ -295,19 +304,38 @@ __global__ __launch_bounds__(64) void prefill_qkv_epilogue_kernel(bf16_t* qkv, c
     const int q_width = query_heads * kDim;
     const int kv_width = key_value_heads * kDim;
     const int position = first + row;
-    bf16_t* base = qkv + static_cast<size_t>(row) * (q_width + 2 * kv_width) + static_cast<size_t>(head) * kDim;
+    const size_t offset = static_cast<size_t>(row) * (q_width + 2 * kv_width) + static_cast<size_t>(head) * kDim;
+    bf16_t* base = qkv + offset;
+    const bf16_t* projected = base;
+    if constexpr (kSliced) {
+        const float* p = partial + offset + lane;
+        float v[2][8];
+#pragma unroll
+        for (int s = 0; s < 8; ++s)
+            if (s < slices) v[0][s] = p[s * slice], v[1][s] = p[s * slice + 64];
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            float sum = v[i][0];
+#pragma unroll
+            for (int s = 1; s < 8; ++s)
+                if (s < slices) sum += v[i][s];
+            head_lds[lane + 64 * i] = f2bf(sum);
+        }
+        __syncthreads();
+        projected = head_lds;
+    }
     if (head >= query_heads + key_value_heads) {
         const int vh = head - query_heads - key_value_heads;
         for (int d = lane; d < kDim; d += 64) {
             const size_t index = ((static_cast<size_t>(vh) * (value_stride >> 3) + (position >> 3)) * kDim + d) * 8 +
                                  (position & 7);
-            value_cache[index] = base[d];
+            value_cache[index] = projected[d];
         }
         return;
     }
     const bool is_query = head < query_heads;
     bf16_t out0, out1;
-    head_detail::norm_rope_head(base, is_query ? q_norm : k_norm, rope_table + static_cast<size_t>(position) * kDim,
+    head_detail::norm_rope_head(projected, is_query ? q_norm : k_norm, rope_table + static_cast<size_t>(position) * kDim,
                                 epsilon, out0, out1);
     base[lane] = out0;
     base[lane + 64] = out1;
@@ -462,12 +490,17 @@ hipError_t launch_causal_softmax(bf16_t* scores, int heads, int rows, int stride
 
 hipError_t launch_prefill_qkv_epilogue(bf16_t* qkv, const bf16_t* q_norm, const bf16_t* k_norm, const bf16_t* rope_table,
                                        bf16_t* key_cache, bf16_t* value_cache, int value_stride, int first, int rows,
-                                       int query_heads, int key_value_heads, float epsilon, hipStream_t stream) {
-    if (rows <= 0 || query_heads <= 0 || key_value_heads <= 0 || value_stride % 8 != 0) return hipErrorInvalidValue;
+                                       int query_heads, int key_value_heads, float epsilon, const float* partial,
+                                       int slices, hipStream_t stream) {
+    if (rows <= 0 || query_heads <= 0 || key_value_heads <= 0 || value_stride % 8 != 0 || slices < 1 || slices > 8 ||
+        (slices > 1 && partial == nullptr)) {
+        return hipErrorInvalidValue;
+    }
     const int heads = query_heads + 2 * key_value_heads;
-    prefill_qkv_epilogue_kernel<<<rows * heads, 64, 0, stream>>>(qkv, q_norm, k_norm, rope_table, key_cache, value_cache,
-                                                                 value_stride, first, query_heads, key_value_heads,
-                                                                 epsilon);
+    const size_t slice = static_cast<size_t>(rows) * heads * 128;
+    const auto kernel = slices > 1 ? prefill_qkv_epilogue_kernel<true> : prefill_qkv_epilogue_kernel<false>;
+    kernel<<<rows * heads, 64, 0, stream>>>(qkv, q_norm, k_norm, rope_table, key_cache, value_cache, value_stride, first,
+                                            query_heads, key_value_heads, epsilon, partial, slices, slice);
     return hipGetLastError();
 }
 

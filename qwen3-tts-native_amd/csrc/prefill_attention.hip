@@ -278,8 +278,11 @@ hipError_t launch_prefill_attention(const bf16_t* qkv, int qkv_width, const bf16
     }
     const float scale = 1.0f / sqrtf(static_cast<float>(head_dimension));
     const int tiles = (rows + kRows - 1) / kRows;
-    // two heads of a key/value head share its key and value loads
-    if (query_heads / key_value_heads % 2 == 0) {
+    // two heads of a key/value head share its key and value loads, once blocks
+    // of one head would outnumber the 256 CUs; below, latency alone counts and
+    // a block of one head has half the exponentials in its chain (33 rows, two
+    // heads 10.8 us a layer).  A head's arithmetic is the same either way.
+    if (query_heads / key_value_heads % 2 == 0 && tiles * query_heads > 256) {
         prefill_attention_kernel<2><<<dim3(tiles, query_heads / 2), 64 * kWaves, 0, stream>>>(
             qkv, qkv_width, key_cache, value_cache, value_stride, out, rows, query_heads, key_value_heads, scale);
     } else {

@@ -482,6 +482,10 @@ struct Bf16GemmArgs {
     const bf16_t* norm_weight = nullptr;
     bf16_t* norm_out = nullptr;
     float norm_epsilon = 0.f;
+    // kGemmStore through launch_gemm_dma: where K is sliced, leave the slices
+    // in `partial` ([slice][m][n]), C unwritten, and store their count here
+    // (untouched where C is written); host memory, or null
+    int* open_slices = nullptr;
 };
 hipError_t launch_bf16_gemm(const Bf16GemmArgs& args, hipStream_t stream);
 // The same products through direct-to-LDS loads (gemm_dma.hip): unbatched, K a
@@ -503,7 +507,8 @@ hipError_t launch_causal_softmax(bf16_t* scores, int heads, int rows, int stride
                                  hipStream_t stream);
 hipError_t launch_prefill_qkv_epilogue(bf16_t* qkv, const bf16_t* q_norm, const bf16_t* k_norm, const bf16_t* rope_table,
                                        bf16_t* key_cache, bf16_t* value_cache, int value_stride, int first, int rows,
-                                       int query_heads, int key_value_heads, float epsilon, hipStream_t stream);
+                                       int query_heads, int key_value_heads, float epsilon, const float* partial,
+                                       int slices, hipStream_t stream);
 // Integers as bf16 (exact: |v| <= 127); count a multiple of 8.
 hipError_t launch_int8_to_bf16(const int8_t* source, bf16_t* destination, size_t count, hipStream_t stream);
 hipError_t launch_prompt_rows(bf16_t* rows_data, const int* text, const int* codec, const bf16_t* codec_embedding,

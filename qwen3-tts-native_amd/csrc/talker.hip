@@ -789,9 +789,12 @@ public:
             g.b2_row = qw;
             g.b3 = L.v16;
             g.b3_row = qw + kvw;
+            int slices = 1;
+            g.open_slices = &slices;  // short prompts slice K; the epilogue adds the slices
             check_hip(launch_bf16_gemm(g, stream_), "prefill q/k/v GEMM");
             check_hip(launch_prefill_qkv_epilogue(qkv, L.q_norm, L.k_norm, m_.rope_table_.as<bf16_t>(), kc, vc, vstride, 0,
-                                                  rows, T.query_heads, T.key_value_heads, cfg_.eps, stream_),
+                                                  rows, T.query_heads, T.key_value_heads, cfg_.eps, g.partial, slices,
+                                                  stream_),
                       "prefill q/k norm + RoPE + cache");
             check_hip(launch_prefill_attention(qkv, qkvw, kc, vc, vstride, attn, rows, T.query_heads, T.key_value_heads, hd,
                                                stream_),
