@@ -65,16 +65,15 @@ __device__ __forceinline__ T* of_stream(T* p, const Streams& st, int s) {
 // ---------------------------------------------------------------------------
 // Rows GEMV for 1..4 rows (transformer projections, RVQ projection, causal
 // pre-convolution).  One wave computes one output channel of one stream
-// (blockIdx.y): its
-// lanes hold the rows in registers (float4 at k = 256 * c + 4 * lane, read
-// from L2), apply RMSNorm there when asked (CS:414-434: each wave reduces the
+// (blockIdx.y): its lanes hold the rows in registers (float4 at k = 256 * c +
+// 4 * lane, read from L2), apply RMSNorm there when asked (CS:414-434: each wave reduces the
 // row's squares itself), stream each channel's weight row with float4 loads
 // and finish with butterfly sums.  No LDS and no barrier: the launch's
 // latency is one weight read plus one reduction (two with the norm), so the
 // rows' sums travel together (wave_sums) and the epilogue's operands are
 // requested beside the weights (a 1-frame packet 590 -> 545 us,
-// 4 frames 757 -> 737 us, six streams 2235 -> 2189 us).  Four channels a block: one wave a block
-// cost the packet about 5 us more.  Matrix-core tiles (16 rows, 4 used) were
+// 4 frames 757 -> 737 us, six streams 2235 -> 2189 us).  Four channels a
+// block: one wave a block cost the packet about 5 us more.  Matrix-core tiles (16 rows, 4 used) were
 // slower here: 512 x 1024 3.3 -> 5.6 us, gate/up 5.2 -> 6.9 us.
 // kRows: 1, 2 or 4, the least that holds the packet's rows.
 // ---------------------------------------------------------------------------
