@@ -865,11 +865,20 @@ int32_t begin_host_group(Qwen3TtsCodecContextV1* const* group, const uint16_t* c
         write_error(error, capacity, "allocate decoder batch workspace");
         return kAlloc;
     }
-    // whatever the other sessions' streams still hold comes first
+    // Whatever the other sessions' streams still hold comes first.  They are
+    // idle except after a call that failed, and an idle stream is left alone:
+    // an event recorded there takes one of the process's four hardware queues,
+    // which other groups' leaders then share (packets of 1, 1, 2, 2, 3 and 3
+    // frames: 2455 us with every member joined, 1735 us so; two 1-frame
+    // packets 664 and 615 us).
     for (int i = 1; i < count && st == hipSuccess; ++i) {
+        st = hipStreamQuery(group[i]->stream);
+        if (st != hipErrorNotReady) continue;
+        (void)hipGetLastError();  // not an error: the launches below ask for theirs
         st = hipEventRecord(group[i]->join_event, group[i]->stream);
         if (st == hipSuccess) st = hipStreamWaitEvent(lead->stream, group[i]->join_event, 0);
     }
+    if (st != hipSuccess) return hip_error(error, capacity, "order decoder streams", st);
     for (int i = 0; i < count && st == hipSuccess; ++i) st = hipEventRecord(group[i]->start_event, lead->stream);
     if (st != hipSuccess) return hip_error(error, capacity, "start packet timing", st);
     constexpr size_t kCodes = kMaxFrames * kCodebooks;
