@@ -71,11 +71,11 @@ struct ConvArgs {
     float* snake_out;
     const float* snake_alpha;
     const float* snake_beta_den;
-    float* partial;  // K slices' sums, [slice][rows of all streams][n]: conv_partial_floats
+    float* partial;  // K slices' sums, [slice][m][n] in each stream's own arena: conv_partial_floats
     Streams streams;
 };
 hipError_t launch_conv(const ConvArgs& args, hipStream_t stream);
-size_t conv_partial_floats(int m, int n, int k, int streams);
+size_t conv_partial_floats(int m, int n, int k);  // of one stream
 
 // ---- rows GEMV (1..4 rows) -------------------------------------------------
 enum RowsEpilogue : int {

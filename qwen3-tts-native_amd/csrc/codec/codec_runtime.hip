@@ -294,8 +294,6 @@ struct Qwen3TtsCodecContextV1 {
     float *cur[4] = {}, *ext2[4] = {};
     float *preclamp = nullptr, *clamped = nullptr;
     float* partial = nullptr;
-    // K slices' sums of a batch that this session leads, allocated with its first batch
-    float* batch_partial = nullptr;
     CopySegment* seg_in[kMaxFrames + 1] = {};
     CopySegment* seg_out[kMaxFrames + 1] = {};
 
@@ -320,10 +318,11 @@ int segments_for_stop(int stop) {
     }
 }
 
-// K slices' workspace: the largest over the packet's products and frame counts
-size_t partial_floats(int streams) {
+// K slices' workspace: the largest over the packet's products and frame
+// counts.  A batch uses each member's own, so it needs no other.
+size_t partial_floats() {
     size_t most = 0;
-    auto add = [&](int m, int n, int k) { most = std::max(most, conv_partial_floats(m, n, k, streams)); };
+    auto add = [&](int m, int n, int k) { most = std::max(most, conv_partial_floats(m, n, k)); };
     for (int f = 1; f <= kMaxFrames; ++f) {
         for (int u = 0; u < 2; ++u) {
             const int m = f << u;  // 1x / 2x frames in, then 2x / 4x after the transposed conv
@@ -389,7 +388,7 @@ void layout_session(Qwen3TtsCodecContextV1* s, Arena& a) {
     s->preclamp = a.take<float>((size_t)F * kSamplesPerFrame);
     s->clamped = a.take<float>((size_t)F * kSamplesPerFrame);
     s->history_bytes = hist;
-    s->partial = a.take<float>(std::max<size_t>(partial_floats(1), 1));
+    s->partial = a.take<float>(std::max<size_t>(partial_floats(), 1));
     for (int f = 0; f <= kMaxFrames; ++f) {
         s->seg_in[f] = a.take<CopySegment>(kSegments);
         s->seg_out[f] = a.take<CopySegment>(kSegments);
@@ -458,15 +457,14 @@ struct Launcher {
     const Weights& w;
     Streams streams;
     PcmTargets pcm;
-    float* partial;
     hipError_t st = hipSuccess;
 
-    explicit Launcher(Qwen3TtsCodecContextV1* one) : s(one), w(one->model->w), pcm{}, partial(one->partial) {
+    explicit Launcher(Qwen3TtsCodecContextV1* one) : s(one), w(one->model->w), pcm{} {
         pcm.pcm[0] = one->mapped_pcm;
     }
     // sessions of one model, each on its own arena
     Launcher(Qwen3TtsCodecContextV1* const* group, int count)
-        : s(group[0]), w(group[0]->model->w), pcm{}, partial(group[0]->batch_partial) {
+        : s(group[0]), w(group[0]->model->w), pcm{} {
         streams.count = count;
         for (int i = 0; i < count; ++i) {
             streams.delta[i] = static_cast<char*>(group[i]->arena) - static_cast<char*>(group[0]->arena);
@@ -505,7 +503,7 @@ struct Launcher {
         g.snake_out = snake_out;
         g.snake_alpha = alpha;
         g.snake_beta_den = beta;
-        g.partial = partial;
+        g.partial = s->partial;
         g.streams = streams;
         ok(launch_conv(g, s->stream));
     }
@@ -858,13 +856,6 @@ int32_t begin_host_group(Qwen3TtsCodecContextV1* const* group, const uint16_t* c
     Qwen3TtsCodecContextV1* lead = group[0];
     hipError_t st = hipSetDevice(lead->device);
     if (st != hipSuccess) return hip_error(error, capacity, "select HIP device", st);
-    if (!lead->batch_partial &&
-        hipMalloc(reinterpret_cast<void**>(&lead->batch_partial),
-                  std::max<size_t>(partial_floats(kMaxStreams), 1) * sizeof(float)) != hipSuccess) {
-        lead->batch_partial = nullptr;
-        write_error(error, capacity, "allocate decoder batch workspace");
-        return kAlloc;
-    }
     // Whatever the other sessions' streams still hold comes first.  They are
     // idle except after a call that failed, and an idle stream is left alone:
     // an event recorded there takes one of the process's four hardware queues,
@@ -930,7 +921,6 @@ void release_context(Qwen3TtsCodecContextV1* s) {
     for (auto& g : s->graphs)
         if (g) (void)hipGraphExecDestroy(g);
     if (s->arena) (void)hipFree(s->arena);
-    if (s->batch_partial) (void)hipFree(s->batch_partial);
     if (s->host_pcm) (void)hipHostFree(s->host_pcm);
     if (s->host_codes) (void)hipHostFree(s->host_codes);
     if (s->start_event) (void)hipEventDestroy(s->start_event);

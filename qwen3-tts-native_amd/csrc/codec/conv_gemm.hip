@@ -349,7 +349,8 @@ __global__ __launch_bounds__(64 * kWM * kWN * kWK) void tile_kernel(ConvArgs g, 
             const int col = n0 + wn + 16 * j + 4 * group;
             if (col >= g.n) continue;
             if (slices > 1)
-                *reinterpret_cast<floatx4*>(g.partial + (static_cast<size_t>(blockIdx.y) * rows + r) * g.n + col) = acc[i][j];
+                *reinterpret_cast<floatx4*>(g.partial + at.delta + (static_cast<size_t>(blockIdx.y) * g.m + at.p) * g.n + col) =
+                    acc[i][j];
             else
                 store_epilogue(g, at, col, kAhead ? ein : load_epilogue(g, at, col, col % g.channels_out), acc[i][j]);
         }
@@ -365,8 +366,8 @@ __global__ __launch_bounds__(64) void reduce_kernel(ConvArgs g, int slices) {
     const int r = t / quads, col = (t - r * quads) * 4;
     const Row at = locate(g, r);
     const EpilogueIn e = load_epilogue(g, at, col, col % g.channels_out);
-    const size_t slice = static_cast<size_t>(rows) * g.n;
-    const float* p = g.partial + static_cast<size_t>(r) * g.n + col;
+    const size_t slice = static_cast<size_t>(g.m) * g.n;
+    const float* p = g.partial + at.delta + static_cast<size_t>(at.p) * g.n + col;
     floatx4 sum = load4(p);
     for (int z0 = 1; z0 < slices; z0 += 4) {  // four slices' loads in flight
         floatx4 v[4];
@@ -453,9 +454,9 @@ bool valid(const ConvArgs& g) {
 
 }  // namespace
 
-size_t conv_partial_floats(int m, int n, int k, int streams) {
+size_t conv_partial_floats(int m, int n, int k) {
     const Summation how = summation(m, n, k);
-    return how.slices > 1 ? static_cast<size_t>(how.slices) * m * streams * n : 0;
+    return how.slices > 1 ? static_cast<size_t>(how.slices) * m * n : 0;
 }
 
 hipError_t launch_conv(const ConvArgs& g, hipStream_t stream) {

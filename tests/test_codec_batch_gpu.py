@@ -1,6 +1,8 @@
 """Packets of several streams that share their launches: each stream's PCM is
 the bits it gets alone, whatever the other streams' packet sizes, and every
 packet size agrees with the float64 whole-utterance model."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -64,3 +66,24 @@ def test_packet_size_matches_float64(model, weights, frames):
     s = model.session()
     got = np.concatenate([s.debug_checkpoint(codes[at:at + frames], 12, 1920 * frames, 1) for at in (0, frames)])
     assert np.abs(got - whole[12]).max() <= 5e-6 * max(1.0, np.abs(whole[12]).max())
+
+
+def test_batches_allocate_no_device_memory(codec, model):
+    """A batch works in its members' own memory: sessions that lead their
+    first batch (of several packet sizes, and of one) leave the device's free
+    memory as it was, and report the same bytes as before."""
+    hip = C.CDLL("libamdhip64.so")
+    sessions = [model.session() for _ in range(6)]
+    streams = [M.random_codes(12, 70 + i) for i in range(6)]
+    # the launches' own first-use allocations, on other sessions' buffers
+    codec.process_batch([model.session() for _ in range(2)], [s[:4] for s in streams[:2]])
+    before = [s.memory().device_bytes for s in sessions]
+    free, after, total = C.c_size_t(), C.c_size_t(), C.c_size_t()
+    assert hip.hipMemGetInfo(C.byref(free), C.byref(total)) == 0
+    for order in (range(6), reversed(range(6))):
+        order = list(order)
+        codec.process_batch([sessions[i] for i in order], [streams[i][:4] for i in order])
+    codec.process_batch(sessions, [streams[i][8:8 + 1 + i // 2] for i in range(6)])
+    assert hip.hipMemGetInfo(C.byref(after), C.byref(total)) == 0
+    assert after.value == free.value
+    assert [s.memory().device_bytes for s in sessions] == before
