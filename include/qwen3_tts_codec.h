@@ -275,11 +275,15 @@ QWEN3_TTS_CODEC_API int32_t qwen3_tts_codec_process_packet_v1(Qwen3TtsCodecConte
                                                               size_t pcm_capacity_samples,
                                                               Qwen3TtsCodecPacketResultV1* result, char* error,
                                                               size_t error_capacity);
-/* Items are validated and queued in array order; the first failure ends the
- * batch and is returned, and the items before it still complete.  Every
- * item's result is cleared on entry, so after an error the items whose packet
- * completed (and advanced their stream) are exactly those with a nonzero
- * result->frame_count. */
+/* Items are validated in array order; the first bad one ends the batch and is
+ * returned, and the items before it still complete.  Items of one model with
+ * equal frame_count share one sequence of launches, queued in the order of
+ * their first items; where one fails to queue, its items fail together (their
+ * sessions need a reset) and nothing is queued after it, while what was queued
+ * before still completes.  gpu_microseconds of an item is the time of the
+ * launches it shared.  Every item's result is cleared on entry, so after an
+ * error the items whose packet completed (and advanced their stream) are
+ * exactly those with a nonzero result->frame_count. */
 QWEN3_TTS_CODEC_API int32_t qwen3_tts_codec_process_batch_v1(Qwen3TtsCodecBatchItemV1* items, uint32_t item_count,
                                                              char* error, size_t error_capacity);
 

@@ -299,6 +299,7 @@ struct Qwen3TtsCodecContextV1 {
 
     hipGraphExec_t graphs[kMaxFrames + 1] = {};
     bool use_graphs = true;
+    bool fail_group = false;  // test switch: a batch that this session leads fails behind its launches
 };
 
 namespace {
@@ -880,9 +881,16 @@ int32_t begin_host_group(Qwen3TtsCodecContextV1* const* group, const uint16_t* c
     if (st != hipSuccess) return hip_error(error, capacity, "upload frontend codes", st);
     Launcher l(group, count);
     l.packet((int)frames, 0);
-    if (l.st != hipSuccess) return hip_error(error, capacity, "launch decoder packet", l.st);
-    for (int i = 0; i < count && st == hipSuccess; ++i) st = hipEventRecord(group[i]->stop_event, lead->stream);
-    return st == hipSuccess ? kOk : hip_error(error, capacity, "record packet completion", st);
+    if (lead->fail_group) l.ok(hipErrorLaunchFailure);
+    if (l.st == hipSuccess)
+        for (int i = 0; i < count && st == hipSuccess; ++i) st = hipEventRecord(group[i]->stop_event, lead->stream);
+    if (l.st == hipSuccess && st == hipSuccess) return kOk;
+    // Some of the launches may have advanced the members' device state, none
+    // of which the host has counted: they need a reset, as after a device
+    // packet that failed to queue.
+    for (int i = 0; i < count; ++i) group[i]->cancelled = true;
+    return l.st != hipSuccess ? hip_error(error, capacity, "launch decoder packet", l.st)
+                              : hip_error(error, capacity, "record packet completion", st);
 }
 
 int32_t check_packet_args(Qwen3TtsCodecContextV1* s, const uint16_t* codes, uint32_t frames, int32_t is_final,
@@ -969,6 +977,8 @@ int32_t create_context(int32_t device, Qwen3TtsCodecModelV1* model, bool shared_
     if (shared_session) model->active_sessions.fetch_add(1, std::memory_order_acq_rel);
     const char* graphs = std::getenv("QWEN3_TTS_CODEC_GRAPH");
     s->use_graphs = !(graphs && graphs[0] == '0');
+    const char* fail_group = std::getenv("QWEN3_TTS_CODEC_TEST_FAIL_GROUP");
+    s->fail_group = fail_group && fail_group[0] == '1';
     st = hipStreamCreateWithFlags(&s->stream, hipStreamNonBlocking);
     if (st == hipSuccess) st = hipEventCreate(&s->start_event);
     if (st == hipSuccess) st = hipEventCreate(&s->stop_event);
@@ -1457,8 +1467,9 @@ QWEN3_TTS_CODEC_API int32_t qwen3_tts_codec_process_batch_v1(Qwen3TtsCodecBatchI
     }
     // Items are checked in order; those before the first bad one are decoded.
     // Packets of equal length on one model run as one sequence of launches,
-    // different groups side by side on their first session's streams, and all
-    // are queued before any is waited for.  The first failure is reported.
+    // different groups side by side on their first session's streams, queued
+    // in the order of their first items before any is waited for; a group that
+    // fails ends the queueing.  The first failure is reported.
     // Results are cleared first: after a failed batch, an item whose packet
     // completed (and advanced its stream) is the one whose result has a
     // nonzero frame_count.
@@ -1499,6 +1510,7 @@ QWEN3_TTS_CODEC_API int32_t qwen3_tts_codec_process_batch_v1(Qwen3TtsCodecBatchI
         } else {
             (void)hipStreamSynchronize(group[0]->stream);  // no launch of a failed group outlives the call
             if (status == kOk) status = r;
+            break;
         }
     }
     for (uint32_t i = 0; i < checked; ++i) {

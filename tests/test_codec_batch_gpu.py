@@ -87,3 +87,44 @@ def test_batches_allocate_no_device_memory(codec, model):
     assert hip.hipMemGetInfo(C.byref(after), C.byref(total)) == 0
     assert after.value == free.value
     assert [s.memory().device_bytes for s in sessions] == before
+
+
+def test_failed_launches_cancel_their_members_alone(codec, model, monkeypatch):
+    """Shared launches that fail to queue (forced on the leader, behind its
+    launches) fail all their items, whose sessions then refuse packets until a
+    reset; what was queued before completes, what comes after is not begun and
+    goes on where it was."""
+    def leader():
+        with monkeypatch.context() as m:
+            m.setenv("QWEN3_TTS_CODEC_TEST_FAIL_GROUP", "1")
+            return model.session()
+
+    sessions = [model.session(), leader(), model.session(), model.session()]
+    sizes = [1, 3, 2, 3]  # launched as (0), (1, 3), (2)
+    streams = [M.random_codes(8, 80 + i) for i in range(4)]
+    for s, c in zip(sessions, streams):
+        s.packet(c[:4])
+    results = [codec.PacketResult() for _ in sessions]
+    pcms = [np.zeros(7680, np.int16) for _ in sessions]
+    items = (codec.BatchItem * 4)()
+    parts = [np.ascontiguousarray(c[4:4 + n]) for c, n in zip(streams, sizes)]
+    for i, s in enumerate(sessions):
+        items[i] = codec.BatchItem(s.handle, parts[i].ctypes.data, sizes[i], 0, pcms[i].ctypes.data, 7680,
+                                   C.pointer(results[i]))
+    with pytest.raises(codec.CodecError) as e:
+        codec.call("qwen3_tts_codec_session_process_batch_v1", items, 4)
+    assert e.value.status == -2 and "launch decoder packet" in e.value.message
+    assert [r.frame_count for r in results] == [1, 0, 0, 0]
+    assert [s.state().frame_position for s in sessions] == [5, 4, 4, 4]
+    for i in (1, 3):
+        with pytest.raises(codec.CodecError) as e:
+            sessions[i].packet(parts[i])
+        assert e.value.status == -3
+        sessions[i].reset()
+    for i, (s, c) in enumerate(zip(sessions, streams)):
+        alone = model.session()
+        want = [alone.packet(c[:4])[0], alone.packet(parts[i])[0]]
+        if i in (1, 3):
+            assert np.array_equal(s.packet(c[:4])[0], want[0])
+        got = pcms[i][:1920] if i == 0 else s.packet(parts[i])[0]
+        assert np.array_equal(got, want[1]), i
