@@ -76,6 +76,10 @@ void orc_expf_array(const float* in, float* out, size_t n) {
     for (size_t i = 0; i < n; ++i) out[i] = q3_expf(in[i]);
 }
 
+void orc_expf_nonpositive_array(const float* in, float* out, size_t n) {
+    for (size_t i = 0; i < n; ++i) out[i] = q3_expf_nonpositive(in[i]);
+}
+
 static inline float bf(uint16_t v) { return orc_bf16_to_f32(v); }
 static inline uint16_t tobf(float f) { return orc_f32_to_bf16(f); }
 static inline float rbf(float f) { return bf(tobf(f)); }

@@ -32,6 +32,7 @@ void orc_bf16_to_f32_array(const uint16_t* in, float* out, size_t n);
 uint64_t orc_xorshift64star(uint64_t* state);
 /* q3_expf (the exp shared with the HIP kernels) over an array. */
 void orc_expf_array(const float* in, float* out, size_t n);
+void orc_expf_nonpositive_array(const float* in, float* out, size_t n);
 float orc_uniform_random(uint64_t* state);
 
 /* ---- int8 GEMV family (K/int8_gemv.cu) --------------------------------- */

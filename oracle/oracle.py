@@ -201,6 +201,13 @@ def expf_array(x):
     return out
 
 
+def expf_nonpositive_array(x):
+    x = _c(x, np.float32)
+    out = np.empty_like(x)
+    lib().orc_expf_nonpositive_array(_p(x), _p(out), C.c_size_t(x.size))
+    return out
+
+
 def set_threads(threads: int) -> None:
     """Threads for the model-level GEMVs of large matrices (bit-identical
     results for any count)."""

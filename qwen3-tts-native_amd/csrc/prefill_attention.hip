@@ -18,11 +18,14 @@
 // in which the value cache holds 8 positions of one dimension.  So neither
 // probabilities nor values move through LDS or a transposed copy.
 //
-// Bound by the exponentials (q3_expf, 16 of them per lane and key block) and
-// the latency of a block's loads.  Per layer, 16 query and 8 key/value heads:
+// Bound by the exponentials (16 of them per lane, head and key block; q3_expf's
+// bits: the hardware's exp2 with a first-order correction, 0.41 ulp rms against
+// q3_expf's 0.30, saved 0.8 us of 16 at 512 rows) and the latency of a block's
+// loads.  Per layer, 16 query and 8 key/value heads:
 // 512 rows (score GEMM, softmax, value transpose, value GEMM) 60 us, 801 rows
 // (per-row chains) 291 us before; now 16 and 33 us (33 rows, latency alone: 10 us).
 #include "q3_common.hpp"
+#include "q3_math.h"
 
 namespace q3 {
 namespace {
@@ -34,17 +37,6 @@ constexpr int kDim = 128;
 constexpr int kRows = 16;   // query rows of a block
 constexpr int kKeys = 32;   // keys of a step
 constexpr int kWaves = 4;
-
-// exp(x) for x <= 0 to about an ulp: the hardware's 2^t at t = x log2(e), and
-// the rounding of t put back in first order.  -inf gives 0, NaN stays.
-__device__ __forceinline__ float exp_below(float x) {
-    constexpr float kLog2e = 1.44269504088896341f, kLog2eLow = 1.92596299e-8f, kLn2 = 0.693147180559945309f;
-    x = x < -200.f ? -200.f : x;
-    const float t = x * kLog2e;
-    const float low = fmaf(x, kLog2eLow, fmaf(x, kLog2e, -t));
-    const float e = __builtin_amdgcn_exp2f(t);
-    return fmaf(e, low * kLn2, e);
-}
 
 // Two floats to a pair of bf16 (nearest even) in one word, and back.
 __device__ __forceinline__ unsigned pack(float lo, float hi) {
@@ -58,7 +50,8 @@ __device__ __forceinline__ float high_of(unsigned w) { return __uint_as_float(w 
 __device__ __forceinline__ bf16x8_t load8(const bf16_t* p) { return *reinterpret_cast<const bf16x8_t*>(p); }
 
 template <int kHeads>
-__global__ __launch_bounds__(64 * kWaves) void prefill_attention_kernel(const bf16_t* qkv, int qkv_width,
+// Two waves a SIMD: unbounded, the compiler takes 1 us more (512 rows 16.9, now 16.2).
+__global__ __launch_bounds__(64 * kWaves, 2) void prefill_attention_kernel(const bf16_t* qkv, int qkv_width,
                                                                          const bf16_t* key_cache,
                                                                          const bf16_t* value_cache, int value_stride,
                                                                          bf16_t* out, int rows, int query_heads,
@@ -101,11 +94,21 @@ __global__ __launch_bounds__(64 * kWaves) void prefill_attention_kernel(const bf
     auto scores = [&](const bf16x8_t (&kf)[2][4], unsigned (&s)[kHeads][4]) {
 #pragma unroll
         for (int h = 0; h < kHeads; ++h) {
-            floatx4_t acc[2] = {floatx4_t{0.f, 0.f, 0.f, 0.f}, floatx4_t{0.f, 0.f, 0.f, 0.f}};
+            // two chains of two, not one of four: error of the 128 products'
+            // sum, rms in 2^-24 of the sums', 0.84 against 1.00 (0.80 as the
+            // exact kernels' tree; four products added: 0.80 too, but 8 us more
+            // of 32 at 801 rows)
+            floatx4_t acc[2];
 #pragma unroll
-            for (int kk = 0; kk < 4; ++kk)
+            for (int t = 0; t < 2; ++t) {
+                floatx4_t half[2];
 #pragma unroll
-                for (int t = 0; t < 2; ++t) acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[t][kk], qf[h][kk], acc[t], 0, 0, 0);
+                for (int i = 0; i < 2; ++i) {
+                    half[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[t][2 * i], qf[h][2 * i], floatx4_t{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+                    half[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[t][2 * i + 1], qf[h][2 * i + 1], half[i], 0, 0, 0);
+                }
+                acc[t] = half[0] + half[1];
+            }
 #pragma unroll
             for (int t = 0; t < 2; ++t)
 #pragma unroll
@@ -138,11 +141,11 @@ __global__ __launch_bounds__(64 * kWaves) void prefill_attention_kernel(const bf
                 top = 2 * w <= visible ? fmaxf(top, low_of(s[h][w])) : top;
                 top = 2 * w + 1 <= visible ? fmaxf(top, high_of(s[h][w])) : top;
             }
-            float add = sum[h] == 0.f ? 0.f : sum[h] * exp_below(maximum[h] - top);
+            float add = sum[h] == 0.f ? 0.f : sum[h] * q3_expf_nonpositive(maximum[h] - top);
 #pragma unroll
             for (int w = 0; w < 4; ++w) {
-                add += 2 * w <= visible ? exp_below(low_of(s[h][w]) - top) : 0.f;
-                add += 2 * w + 1 <= visible ? exp_below(high_of(s[h][w]) - top) : 0.f;
+                add += 2 * w <= visible ? q3_expf_nonpositive(low_of(s[h][w]) - top) : 0.f;
+                add += 2 * w + 1 <= visible ? q3_expf_nonpositive(high_of(s[h][w]) - top) : 0.f;
             }
             sum[h] = add;
             maximum[h] = top;
@@ -166,8 +169,8 @@ __global__ __launch_bounds__(64 * kWaves) void prefill_attention_kernel(const bf
         for (int d = 16; d < 64; d <<= 1) {
             const float other_max = __shfl_xor(maximum[h], d, 64), other_sum = __shfl_xor(sum[h], d, 64);
             const float top = fmaxf(maximum[h], other_max);
-            const float mine = sum[h] == 0.f ? 0.f : sum[h] * exp_below(maximum[h] - top);
-            const float theirs = other_sum == 0.f ? 0.f : other_sum * exp_below(other_max - top);
+            const float mine = sum[h] == 0.f ? 0.f : sum[h] * q3_expf_nonpositive(maximum[h] - top);
+            const float theirs = other_sum == 0.f ? 0.f : other_sum * q3_expf_nonpositive(other_max - top);
             sum[h] = mine + theirs;
             maximum[h] = top;
         }
@@ -184,7 +187,7 @@ __global__ __launch_bounds__(64 * kWaves) void prefill_attention_kernel(const bf
 #pragma unroll
         for (int w = 0; w < kWaves; ++w) {
             const float part_sum = sum_lds[w][h][m];
-            total += part_sum == 0.f ? 0.f : part_sum * exp_below(max_lds[w][h][m] - top);
+            total += part_sum == 0.f ? 0.f : part_sum * q3_expf_nonpositive(max_lds[w][h][m] - top);
         }
         maximum[h] = top;
         inverse[h] = 1.0f / total;
@@ -207,8 +210,8 @@ __global__ __launch_bounds__(64 * kWaves) void prefill_attention_kernel(const bf
             unsigned pw[4];
 #pragma unroll
             for (int w = 0; w < 4; ++w) {
-                const float lo = exp_below(low_of(s[h][w]) - maximum[h]) * inverse[h];
-                const float hi = exp_below(high_of(s[h][w]) - maximum[h]) * inverse[h];
+                const float lo = q3_expf_nonpositive(low_of(s[h][w]) - maximum[h]) * inverse[h];
+                const float hi = q3_expf_nonpositive(high_of(s[h][w]) - maximum[h]) * inverse[h];
                 pw[w] = pack(2 * w <= visible ? lo : 0.f, 2 * w + 1 <= visible ? hi : 0.f);
             }
             pf[h] = __builtin_bit_cast(bf16x8_t, uint4{pw[0], pw[1], pw[2], pw[3]});

@@ -51,4 +51,23 @@ Q3_FN float q3_expf(float x) {
     return x != x ? x : ranged;
 }
 
+/* q3_expf for x <= 0, with its bits and fewer operations: without the upper
+ * special case, and one ldexp (2^n never overflows; the result is rounded once
+ * either way).  NaN stays NaN. */
+Q3_FN float q3_expf_nonpositive(float x) {
+    const float n = rintf(x * 1.44269504088896341f);
+    float r = fmaf(-n, 0.693145751953125f, x);
+    r = fmaf(-n, 1.42860682030941723e-6f, r);
+    float p = 1.98412698412698413e-4f;
+    p = fmaf(p, r, 1.38888888888888889e-3f);
+    p = fmaf(p, r, 8.33333333333333333e-3f);
+    p = fmaf(p, r, 4.16666666666666667e-2f);
+    p = fmaf(p, r, 1.66666666666666667e-1f);
+    p = fmaf(p, r, 0.5f);
+    p = fmaf(p, r, 1.0f);
+    p = fmaf(p, r, 1.0f);
+    const float v = ldexpf(p, (int)fmaxf(n, -400.0f));
+    return x < -103.97208f ? 0.0f : v;
+}
+
 #endif

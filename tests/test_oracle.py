@@ -259,6 +259,21 @@ def test_expf_within_one_ulp(orc):
     assert orc.expf_array(np.array([np.inf, -np.inf, 100.0, -200.0], np.float32)).tolist() == [np.inf, 0.0, np.inf, 0.0]
 
 
+def test_expf_nonpositive_has_expf_bits(orc):
+    """The prompt attention's exponential of scores below their maximum is the
+    common one, bit for bit: around the range's ends, over its middle, -inf; NaN stays NaN."""
+    r = np.random.default_rng(4)
+    edge = np.float32(-103.97208).view(np.uint32)
+    near = np.arange(edge - 5000, edge + 5000, dtype=np.uint32).view(np.float32)  # where results vanish
+    small = np.arange(0x80000000, 0x80000000 + 5000, dtype=np.uint32).view(np.float32)  # -0 and subnormals
+    x = np.concatenate([near, small, -np.exp(r.uniform(-30, 6, 1_000_000)).astype(np.float32),
+                        r.uniform(-110, 0, 1_000_000).astype(np.float32),
+                        -np.arange(20000, dtype=np.float32) / 128,
+                        np.array([0.0, -0.0, -np.inf, -3.4e38, -1e4], np.float32)])
+    assert np.array_equal(orc.expf_nonpositive_array(x).view(np.uint32), orc.expf_array(x).view(np.uint32))
+    assert np.isnan(orc.expf_nonpositive_array(np.array([np.nan], np.float32)))[0]
+
+
 # ---------------------------------------------------------------------------
 # sampler
 # ---------------------------------------------------------------------------
