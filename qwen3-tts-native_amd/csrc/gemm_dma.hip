@@ -465,7 +465,7 @@ hipError_t launch_plain(const Bf16GemmArgs& g, hipStream_t stream) {
             const int splits = std::max(1, std::min(most, 256 / tiles(128, 128)));
             return launch_tile<128, 128, 2, 4, 3, kEpilogue>(g, splits, stream);
         }
-        auto splits = [&](int t) { return std::max(1, std::min(most, (512 + t - 1) / t)); };
+        auto splits = [&](int t) { return g.m > 128 ? most : std::max(1, std::min(most, (512 + t - 1) / t)); };
         if (g.m > 32) return launch_tile<64, 64, 2, 2, 3, kEpilogue>(g, splits(tiles(64, 64)), stream);
         if (g.m > 16) return launch_tile<32, 32, 1, 2, 4, kEpilogue>(g, splits(tiles(32, 32)), stream);
         return launch_tile<16, 32, 1, 2, 4, kEpilogue>(g, splits(tiles(16, 32)), stream);
