@@ -491,24 +491,28 @@ hipError_t launch_plain(const Bf16GemmArgs& g, hipStream_t stream) {
 
 hipError_t launch_gated(const Bf16GemmArgs& g, hipStream_t stream) {
     // Up to 128 rows the weights' stream counts: 32 gate and 32 up columns a
-    // block (6144 + 6144 columns, K 2048: 64 rows 14.6 us, 3.4 TB/s).
+    // block (6144 + 6144 columns, K 2048, random weights from memory: 33 rows
+    // 17.0 us, 64 rows 17.9 us, 2.8 TB/s; 64 x 128 20.6 and 21.3).
     if (g.m <= 16) return launch_tile<16, 64, 1, 2, 4, kGemmGated>(g, 1, stream);
     if (g.m <= 128) return launch_tile<64, 64, 2, 2, 4, kGemmGated>(g, 1, stream);
-    // Beyond: the tile whose rounds over the 256 CUs cost least, by the time
-    // of one block round measured at K 2048 (us; a larger tile reads less and
-    // rounds up more): 512 rows 33.5 with 128 x 192 (one round; 64 x 128
-    // 38.7), 384 27.4 with 96 x 192, 801 56.4 with 64 x 128 (five rounds;
-    // 128 x 192 63.2).
+    // Beyond: the tile whose rounds over the 256 CUs cost least, as a launch
+    // plus a time a round, fitted to all five over 129 to 1152 rows in one run
+    // (us, K 2048, random weights from memory; a larger tile reads less and
+    // rounds up more): 150 rows 24.5 with 96 x 128, 256 26.9 with 128 x 128,
+    // 384 29.8 with 96 x 192, 512 34.8 with 128 x 192 (64 x 128 44.6), 801
+    // 64.8 with 128 x 192 (two rounds; 64 x 128 in five 65.7, 96 x 192 75.8).
+    // The pick is within 1 % of the best up to 1152 rows, 7 % beyond.
     struct Tile {
         int rows, columns;
-        float round;
+        float launch, round;
     };
-    const Tile tile[5] = {{128, 96, 28.5f}, {96, 96, 22.4f}, {128, 64, 19.9f}, {96, 64, 16.6f}, {64, 64, 10.6f}};
+    const Tile tile[5] = {{128, 96, 3.0f, 31.0f}, {96, 96, 3.5f, 25.7f}, {128, 64, 4.0f, 22.0f}, {96, 64, 6.0f, 19.5f},
+                          {64, 64, 6.5f, 11.8f}};
     int best = 0;
     float least = 0.f;
     for (int i = 0; i < 5; ++i) {
         const int blocks = ((g.m + tile[i].rows - 1) / tile[i].rows) * ((g.n + tile[i].columns - 1) / tile[i].columns);
-        const float cost = static_cast<float>((blocks + 255) / 256) * tile[i].round;
+        const float cost = tile[i].launch + static_cast<float>((blocks + 255) / 256) * tile[i].round;
         if (i == 0 || cost < least) {
             best = i;
             least = cost;
