@@ -157,3 +157,51 @@ def test_text_projection_is_as_close_to_exact_as_the_decode_steps(hip, orc, wide
             hip.load().qwen3_tts_session_destroy(s)
     print("values that differ:", [f"{d:.2%}" for d in differ], flush=True)
     assert np.mean(differ) <= 0.0052
+
+
+# Largest distance of a row (2-norm of the difference over the row's).  Sums in
+# another order land on the other side of a rounding step now and then, and one
+# such value early in a row moves many after it: over these prompts any two
+# valid orders (float32, float64 and the device's, its older kernels included)
+# are up to 3.4e-3 (layer 0's caches) and 2.6e-2 (layer 1's, hidden) apart, and
+# 5e-3 over all rows of layer 1.
+# Mistakes planted in the reference, a head of one row taking the row before,
+# 16 gate columns swapped, 64 of the O or down product's K missing, move layer
+# 1's caches by 7e-2 to 0.28 in the worst row, and the columns 2.8e-2 in the
+# median one.
+BOUND = {"layer 0": 2.0 ** -7, "layer 1": 2.0 ** -5, "hidden": 2.0 ** -5}
+OVERALL = 2.0 ** -7
+
+
+# Row counts, by what they are the first (or, one less, the last) to run:
+#  17, 33, 66, 128: K slices in the QKV epilogue, and with the norms; 64-row gate/up tiles to 128
+#  129, 193, 257, 322, 385, 513, 641, 833: the gate/up tiles beyond (all but 64 x 128, which the toy model's widths
+#    take), most ending in a part of a tile
+#  256 / 257: the last prompt of one-head attention blocks and the first of two-head blocks
+#  769, 801: the O product in two slices of 128 x 128 tiles;  1025: unsliced, its norm alone
+#  1409: the text projection on 128 x 128 tiles
+@pytest.mark.parametrize("rows", [17, 33, 66, 128, 129, 193, 256, 257, 322, 385, 513, 641, 769, 801, 833, 1025, 1409])
+def test_wide_prefill_rows(hip, wide, monkeypatch, rows):
+    monkeypatch.delenv("QWEN3_TTS_PREFILL", raising=False)
+    model, reference = wide
+    text, codec = wide_prompt(rows)
+    print(f"wide prefill of {rows} rows", flush=True)
+    s = prefilled(hip, model, text, codec)
+    try:
+        caches, h = reference.run(text, codec)
+        last = np.zeros(WIDE["talker_hidden"], np.uint16)
+        hip.call("qwen3_tts_session_read_last_hidden_v1", s, last.ctypes.data, last.nbytes)
+        pairs = [(f"layer {layer}", read_cache(hip, s, layer, which, rows), caches[layer][which])
+                 for layer in (0, 1) for which in (0, 1)]
+        pairs.append(("hidden", gen.f32(last)[None], reference.norm(h[-1:], "talker.model.norm.weight")))
+        far = {}
+        for what, got, want in pairs:
+            distance = np.linalg.norm(got - want, axis=1) / np.linalg.norm(want, axis=1)
+            row = int(np.argmax(distance))
+            far[what] = max(far.get(what, 0.0), float(distance[row]))
+            assert distance[row] <= BOUND[what], f"{what}, row {row}: {distance[row]:.4g} off"
+            if len(distance) > 1:
+                assert np.sqrt(np.mean(distance ** 2)) <= OVERALL, what
+        print("  largest distances:", {k: f"{v:.2g}" for k, v in far.items()}, flush=True)
+    finally:
+        hip.load().qwen3_tts_session_destroy(s)
