@@ -1069,6 +1069,7 @@ private:
         void ensure(int r, int H, int I, int qkvw, int qw) {
             if (r <= rows) return;
             rows = 0;
+            arena = DeviceBuffer();  // given back before the larger one is taken
             const size_t n = static_cast<size_t>(r);
             size_t used = kPrefillPartialFloats * sizeof(float);
             auto take = [&](size_t elements) {
@@ -1093,8 +1094,8 @@ private:
         int capacity = 0;
         void ensure(int count) {
             if (count <= capacity) return;
-            device = DeviceBuffer(static_cast<size_t>(count) * 2 * sizeof(int));
             release();
+            device = DeviceBuffer(static_cast<size_t>(count) * 2 * sizeof(int));
             check_hip(hipHostMalloc(reinterpret_cast<void**>(&host), static_cast<size_t>(count) * 2 * sizeof(int),
                                     hipHostMallocDefault),
                       "hipHostMalloc(prompt)");
@@ -1103,6 +1104,7 @@ private:
         void release() {
             if (host) (void)hipHostFree(host);
             host = nullptr;
+            device = DeviceBuffer();
             capacity = 0;
         }
     };

@@ -98,3 +98,35 @@ def test_prefill_ignores_an_earlier_prompt(hip, toy, monkeypatch, rows):  # noqa
             hip.load().qwen3_tts_session_destroy(s)
     for fresh, reused in zip(*results):
         assert np.array_equal(fresh, reused)
+
+
+def test_longer_prompts_on_one_session_give_a_fresh_ones_bits(hip, toy, monkeypatch):  # noqa: F811
+    """Prompt and row buffers that grow from prompt to prompt (the old ones
+    are given back first) change nothing."""
+    monkeypatch.delenv("QWEN3_TTS_PREFILL", raising=False)
+    model, _ = toy
+    s = None
+    try:
+        for rows in (5, 70, 33, 290):
+            text, codec = prompt(np.random.default_rng(rows), rows)
+            fresh, want = gpu_prefill(hip, model, 300, text, codec, GREEDY)
+            try:
+                if s is None:
+                    s, got = gpu_prefill(hip, model, 300, text, codec, GREEDY)
+                else:
+                    got = hip.PrefillResult()
+                    p = C.POINTER(C.c_int32)
+                    hip.call("qwen3_tts_session_reset", s, 7)
+                    hip.call("qwen3_tts_session_prefill", s, text.ctypes.data_as(p), codec.ctypes.data_as(p), rows,
+                             hip.SamplingConfig(*GREEDY), C.byref(got))
+                assert got.first_semantic_token == want.first_semantic_token
+                assert np.array_equal(hidden_of(hip, s), hidden_of(hip, fresh))
+                for layer in range(TOY["talker_layers"]):
+                    for which in (0, 1):
+                        assert np.array_equal(read_cache(hip, s, layer, which, rows),
+                                              read_cache(hip, fresh, layer, which, rows))
+            finally:
+                hip.load().qwen3_tts_session_destroy(fresh)
+    finally:
+        if s is not None:
+            hip.load().qwen3_tts_session_destroy(s)
