@@ -170,12 +170,11 @@ __global__ __launch_bounds__(kThreads) void gemv_exact_fixed(GemvArgs a) {
 }
 
 // ---------------------------------------------------------------------------
-// Exact-order rows without the RMSNorm prologue -- 2..8 (exact batched mode)
-// or a whole prompt's (its text projection) -- K = 512 * kVpl known at
-// compile time: the
-// batch-1 kernel's layout -- one unit per half-wave, its weights (the lane's
-// vectors lane + 32 i) requested first and held in registers -- against every
-// input row, staged once per block in LDS.  Per row the sum is the generic
+// Exact-order rows (2..8, the exact batched mode) without the RMSNorm prologue,
+// K = 512 * kVpl known at compile time: the batch-1 kernel's layout -- one unit
+// per half-wave, its weights (the lane's vectors lane + 32 i) requested first
+// and held in registers -- against every input row, staged once per block in
+// LDS.  Per row the sum is the generic
 // kernel's: acc += chain16(vector i) for i in order, then fold32.
 // ---------------------------------------------------------------------------
 template <int kVpl, int kEpi>
@@ -200,42 +199,30 @@ __global__ __launch_bounds__(kThreads) void gemv_exact_rows_fixed(GemvArgs a) {
     }
     __builtin_amdgcn_sched_barrier(0);  // the weight stream first, then the rows
     const uint4* xin = reinterpret_cast<const uint4*>(a.input);
-    // rows in chunks of up to 8 through LDS (more than 8 only for a prompt's
-    // rows: the weights stay in registers for all of them)
-    // gridDim.y groups of rows (a long prompt's rows over more workgroups)
-    const int per_group = (rows + gridDim.y - 1) / gridDim.y;
-    const int r_end = min(rows, static_cast<int>(blockIdx.y + 1) * per_group);
-    for (int r0 = blockIdx.y * per_group; r0 < r_end; r0 += 8) {
-        const int count = min(8, r_end - r0);
-        if (r0 > 0) __syncthreads();  // the previous chunk is read
-        for (int c = threadIdx.x; c < count * kChunks; c += kThreads) {
-            rows_lds[c] = xin[static_cast<size_t>(r0) * kChunks + c];
+    for (int c = threadIdx.x; c < rows * kChunks; c += kThreads) rows_lds[c] = xin[c];
+    __syncthreads();
+    for (int r = 0; r < rows; ++r) {
+        const bf16_t* xs = reinterpret_cast<const bf16_t*>(rows_lds + r * kChunks);
+        float acc[kTiles];
+#pragma unroll
+        for (int t = 0; t < kTiles; ++t) acc[t] = 0.0f;
+#pragma unroll
+        for (int i = 0; i < kVpl; ++i) {
+            float xv[16];
+            load_x16<false>(xs, nullptr, lane + 32 * i, 1.0f, xv);
+#pragma unroll
+            for (int t = 0; t < kTiles; ++t) acc[t] += chain16(w[t][i], xv);
         }
-        __syncthreads();
-        for (int rr = 0; rr < count; ++rr) {
-            const int r = r0 + rr;
-            const bf16_t* xs = reinterpret_cast<const bf16_t*>(rows_lds + rr * kChunks);
-            float acc[kTiles];
 #pragma unroll
-            for (int t = 0; t < kTiles; ++t) acc[t] = 0.0f;
-#pragma unroll
-            for (int i = 0; i < kVpl; ++i) {
-                float xv[16];
-                load_x16<false>(xs, nullptr, lane + 32 * i, 1.0f, xv);
-#pragma unroll
-                for (int t = 0; t < kTiles; ++t) acc[t] += chain16(w[t][i], xv);
-            }
-#pragma unroll
-            for (int t = 0; t < kTiles; ++t) acc[t] = fold32(acc[t]);
-            if (lane == 0 && unit < units) {
-                GemvArgs row = a;
-                row.out16 = a.out16 ? a.out16 + static_cast<size_t>(r) * a.out_features : nullptr;
-                row.out32 = a.out32 ? a.out32 + static_cast<size_t>(r) * a.out_features : nullptr;
-                if constexpr (kSilu) {
-                    store_gate_up<kEpi>(row, unit, acc[0], acc[kTiles - 1]);
-                } else {
-                    store_channel<kEpi>(row, unit, acc[0]);
-                }
+        for (int t = 0; t < kTiles; ++t) acc[t] = fold32(acc[t]);
+        if (lane == 0 && unit < units) {
+            GemvArgs row = a;
+            row.out16 = a.out16 ? a.out16 + static_cast<size_t>(r) * a.out_features : nullptr;
+            row.out32 = a.out32 ? a.out32 + static_cast<size_t>(r) * a.out_features : nullptr;
+            if constexpr (kSilu) {
+                store_gate_up<kEpi>(row, unit, acc[0], acc[kTiles - 1]);
+            } else {
+                store_channel<kEpi>(row, unit, acc[0]);
             }
         }
     }
@@ -248,13 +235,10 @@ hipError_t launch_exact_rows_fixed(const GemvArgs& a, hipStream_t s) {
     const hipError_t st = set_dynamic_lds_once(configured, reinterpret_cast<const void*>(gemv_exact_rows_fixed<kVpl, kEpi>),
                                                static_cast<int>(8 * kIn * sizeof(bf16_t)));
     if (st != hipSuccess) return st;
-    const size_t lds = static_cast<size_t>(std::min(a.rows, 8)) * kIn * sizeof(bf16_t);
-    // more than 8 rows: up to 4 groups of rows on their own workgroups, each
-    // reading the weights again (measured: one workgroup per CU leaves the
-    // per-row arithmetic's latency exposed)
-    const int groups = std::min(4, (a.rows + 7) / 8);
-    const dim3 grid((a.out_features + kHalfWaves - 1) / kHalfWaves, groups);
-    gemv_exact_rows_fixed<kVpl, kEpi><<<grid, kThreads, lds, s>>>(a);
+    if (a.rows < 1 || a.rows > 8) return hipErrorInvalidValue;
+    const size_t lds = static_cast<size_t>(a.rows) * kIn * sizeof(bf16_t);
+    const int blocks = (a.out_features + kHalfWaves - 1) / kHalfWaves;
+    gemv_exact_rows_fixed<kVpl, kEpi><<<blocks, kThreads, lds, s>>>(a);
     return hipGetLastError();
 }
 
