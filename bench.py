@@ -329,10 +329,10 @@ PREFILL_FLOPS_PER_ROW = 2 * 28 * (2048 * 2048 + 2 * 1024 * 2048 + 2048 * 2048 + 
 def prefill_benchmark(hip, rows_list=(96, 512, 801), repeats: int = 5, max_seq: int = 1024):
     """The bf16 prompt prefill through the C ABI at VoiceDesign geometry:
     prompts of `rows_list` positions (96: a short voice-design prompt, whose
-    GEMMs split K; 512: GEMM attention, the largest the reference's GEMM path
-    takes; 801: the exact per-row attention), the
-    median of `repeats` prefills each (qwen3_tts_session_prefill's own GPU
-    time), as prompt positions per second and the GEMMs' TFLOP/s."""
+    GEMMs split K; 512: the largest that the reference's GEMM attention takes;
+    801: beyond, where the reference runs its per-row attention), the median
+    of `repeats` prefills each (qwen3_tts_session_prefill's own GPU time), as
+    prompt positions per second and the GEMMs' TFLOP/s."""
     import numpy as np
 
     lib = hip.load()
@@ -357,7 +357,7 @@ def prefill_benchmark(hip, rows_list=(96, 512, 801), repeats: int = 5, max_seq: 
                 ms = sorted(times[1:])[len(times[1:]) // 2]
                 out[f"rows{rows}"] = {"gpu_ms": round(ms, 3), "positions_per_second": round(rows / (ms * 1e-3), 1),
                                       "gemm_tflops": round(rows * PREFILL_FLOPS_PER_ROW / (ms * 1e-3) / 1e12, 2),
-                                      "attention": "GEMM" if rows <= 512 else "exact per-row kernel"}
+                                      "attention": "one fused launch"}
         finally:
             lib.qwen3_tts_session_destroy(session)
     finally:

@@ -339,9 +339,9 @@ QWEN3_TTS_CODEC_API int32_t qwen3_tts_codec_session_process_packet_v1(
     int16_t* pcm_output, size_t pcm_capacity_samples, Qwen3TtsCodecPacketResultV1* result, char* error,
     size_t error_capacity);
 /* C:433-470: device codes in, producer_ready_event waited on the session's
- * stream, codes snapshotted into the session's ring, codes_consumed_event
- * recorded, the decoder and the pinned PCM copy queued; finish completes the
- * ticket and copies the PCM out. */
+ * stream, codes copied into the session (the device buffer may be written again
+ * behind codes_consumed_event), the decoder queued, whose last kernel writes the
+ * PCM to pinned memory; finish completes the ticket and copies the PCM out. */
 QWEN3_TTS_CODEC_API int32_t qwen3_tts_codec_session_process_device_packet_begin_v2(
     Qwen3TtsCodecSessionV1* session, const Qwen3TtsCodecDevicePacketBeginV2* request,
     Qwen3TtsCodecDevicePacketBeginResultV2* output, char* error, size_t error_capacity);

@@ -402,8 +402,9 @@ QWEN3_TTS_API int32_t qwen3_tts_op_attention(
     uint16_t* const* value_bases, const int32_t* positions, uint16_t* output, int32_t rows,
     int32_t query_heads, int32_t key_value_heads, int32_t head_dimension,
     int32_t max_sequence_length, void* stream, char* error, size_t error_capacity);
-/* The prefill's exact attention for prompts beyond the GEMM path
- * (talker.cu:3035-3054): query rows r = 0..rows-1 against one shared, complete
+/* The reference prefill's exact attention for prompts beyond its GEMM path
+ * (talker.cu:3035-3054; this library's prefill has one kernel for all lengths,
+ * with the same rounding points): query rows r = 0..rows-1 against one shared, complete
  * cache (key_cache and value_cache [capacity][key_value_heads*head_dimension]),
  * row r attending to positions 0..positions[r]; causal_gqa_attention
  * semantics when exact != 0. */
@@ -447,7 +448,7 @@ QWEN3_TTS_API int32_t qwen3_tts_op_decode_attention_noalloc_v1(
     uint16_t* const* value_bases, const int32_t* positions, uint16_t* output, int32_t rows,
     int32_t query_heads, int32_t key_value_heads, int32_t head_dimension,
     int32_t max_sequence_length, void* stream, char* error, size_t error_capacity);
-/* The prefill's bf16 GEMM (the reference's cublasGemmEx / StridedBatchedEx
+/* The bf16 GEMM (the reference prefill's cublasGemmEx / StridedBatchedEx
  * calls with CUBLAS_COMPUTE_32F, talker.cu:2637-2674,2772-2842):
  * C[m][n] = bf16(sum_k A[m][k] * B[n][k]) with fp32 accumulation, all
  * row-major; batch z uses A + z*a_batch, B + (z / b_group)*b_batch and
@@ -466,7 +467,7 @@ QWEN3_TTS_API int32_t qwen3_tts_op_bf16_gemm_v1(
  * are added in slice order.  epilogue 0 stores bf16(sum); 1 adds it into C
  * as add_in_place does after a GEMM (C = bf16(C + bf16(sum))); 2 applies
  * silu_gate with C holding the gate product (C = bf16(bf16(silu(C)) *
- * bf16(sum))).  The prefill uses the planned form. */
+ * bf16(sum))).  The prefill's products run as the planned form does. */
 QWEN3_TTS_API int32_t qwen3_tts_op_bf16_gemm_split_v1(
     const uint16_t* a, const uint16_t* b, uint16_t* c, int32_t m, int32_t n, int32_t k, int32_t lda,
     int32_t ldb, int32_t ldc, int32_t batch, int32_t b_group, int64_t a_batch, int64_t b_batch,

@@ -15,9 +15,10 @@
 //           append, scores, softmax and values fused, with the QKV epilogue.
 //   small   (other caches <= 64 positions) one block of G*128 threads per
 //           (kv head, row), the phases in one kernel.
-// and two for particular callers: prompt-row score tiles (many prompt rows on
-// one shared, complete cache: each key row loaded once for a tile of rows and
-// the heads of its group), and the combine of the batched (non-exact) value
+// and two for particular callers: prompt-row score tiles (the exported prompt
+// attention, many prompt rows on one shared, complete cache: each key row
+// loaded once for a tile of rows and the heads of its group; prefill itself
+// runs prefill_attention.hip), and the combine of the batched (non-exact) value
 // chains when they run as position segments (tolerance mode only).
 //
 // Two arithmetic variants, each the reference's own operation order:
@@ -304,8 +305,9 @@ __global__ __launch_bounds__(kScoreLanes) void attention_scores_kernel(AttnArgs 
 }
 
 
-// Prompt rows against one shared, complete key cache (the prefill's exact
-// attention for long prompts: queries already normalized and rotated):
+// Prompt rows against one shared, complete key cache (the reference's exact
+// attention of long prompts, here an exported op: queries already normalized
+// and rotated):
 // grid (position blocks, kv heads, tiles of kRows rows), one wave, lane =
 // position.  The key row is loaded once for the kRows rows and kG query
 // heads of the tile (the per-row kernel loads it once per row and head).
@@ -1233,7 +1235,7 @@ hipError_t launch_variant(const AttnArgs& a, int rows, hipStream_t stream) {
         attention_small_kernel<kExact, kG><<<dim3(a.key_value_heads, rows), kG * kDim, 0, stream>>>(a);
         return hipGetLastError();
     }
-    // many prompt rows on one complete cache (the prefill's exact attention)
+    // many prompt rows on one complete cache (the exported prompt attention)
     const bool prompt_rows = kExact && a.key_bases == nullptr && a.q_norm == nullptr && rows >= 2 * kPromptTileRows;
     if (prompt_rows) {
         // the key rows are shared

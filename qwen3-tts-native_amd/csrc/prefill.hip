@@ -1,7 +1,11 @@
 // bf16 prompt prefill for gfx950: the reference's prefill runs the talker's
 // bf16 weights through cuBLAS GEMMs with fp32 accumulation and bf16 outputs
 // (native/qwen3-tts-native/native/src/talker.cu:2637-2674, 2750-3249).  Here
-// every such product is one MFMA kernel, gemm_bf16_kernel:
+// its unbatched products of K a multiple of 64, all that a prefill runs, are
+// gemm_dma.hip's and its attention is prefill_attention.hip's.  This file has
+// the prompt rows, the QKV epilogue, the causal softmax (an exported op) and
+// the general product behind the exported GEMMs, gemm_bf16_kernel (batches,
+// any K a multiple of 8, forced plans):
 //
 //   C[m][n] = bf16( sum_k A[m][k] * B[n][k] )      (fp32 accumulation)
 //
@@ -245,7 +249,8 @@ __global__ __launch_bounds__(256) void gemm_bf16_reduce_kernel(Bf16GemmArgs g, i
     gemm_store(g.c + static_cast<size_t>(z) * g.c_batch + static_cast<size_t>(row) * g.ldc + col, sum, g.epilogue);
 }
 
-// causal_softmax_kernel (talker_kernels.cu:232-260) on bf16 scores
+// The exported causal softmax (prefill forms its probabilities in
+// prefill_attention.hip): causal_softmax_kernel (talker_kernels.cu:232-260) on bf16 scores
 // [heads][rows][stride]: scaled = bf16(s * (1/sqrt(d))); maximum over keys
 // 0..query; denominator = sequential fp32 sum of exp(scaled - max); p =
 // bf16(exp(scaled - max) * (1/denominator)); keys query+1 .. stride-1 = 0.

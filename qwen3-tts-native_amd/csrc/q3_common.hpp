@@ -443,7 +443,8 @@ hipError_t launch_sum_embeddings(const bf16_t* const* tables, int count, int voc
 // ldb, a_batch and b_batch must be multiples of 8 and A, B 16-byte aligned.
 // Epilogues of the bf16 GEMM: C = bf16(sum); C = bf16(C + bf16(sum)) (the
 // residual add_in_place); C = bf16(bf16(silu(C)) * bf16(sum)) (silu_gate with
-// C holding the gate product); C = bf16(bf16(sum * scale[n]) + bias[n]), plain
+// C holding the gate product: the exported GEMM's, prefill runs gate and up in
+// one launch); C = bf16(bf16(sum * scale[n]) + bias[n]), plain
 // and with SiLU (the text projection over its int8 weights as bf16 integers).
 enum Bf16GemmEpilogue : int {
     kGemmStore = 0,

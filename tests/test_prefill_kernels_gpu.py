@@ -51,8 +51,9 @@ def hidden_of(hip, s):
     return h
 
 
-# rows at the edges of the gate/up tiles (16, 64, 96, 128) and of the
-# attention's 16 query rows and 32 keys, with one wave to all four at work
+# rows at the edges of this model's gate/up tiles (16 and 64 rows; the others
+# need production widths, test_prefill_widths_gpu.py) and of the attention's 16
+# query rows and 32 keys, with one wave to all four at work
 @pytest.mark.parametrize("rows", [1, 15, 16, 17, 31, 33, 63, 65, 97, 128, 129, 193, 257])
 def test_prefill_matches_oracle_at_tile_edges(hip, orc, toy, monkeypatch, rows):  # noqa: F811
     monkeypatch.delenv("QWEN3_TTS_PREFILL", raising=False)
