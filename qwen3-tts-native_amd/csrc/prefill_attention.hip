@@ -23,7 +23,7 @@
 // q3_expf's 0.30, saved 0.8 us of 16 at 512 rows) and the latency of a block's
 // loads.  Per layer, 16 query and 8 key/value heads:
 // 512 rows (score GEMM, softmax, value transpose, value GEMM) 60 us, 801 rows
-// (per-row chains) 291 us before; now 16 and 33 us (33 rows, latency alone: 10 us).
+// (per-row chains) 291 us before; now 16 and 32 us (33 rows, latency alone: 6 us).
 #include "q3_common.hpp"
 #include "q3_math.h"
 

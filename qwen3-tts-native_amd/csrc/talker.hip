@@ -753,9 +753,9 @@ public:
         };
         // prompt embeddings: int8 text projection, then zero text-less rows
         // and add codec embeddings.  The integers run as bf16 (exactly) on the
-        // matrix cores, scale and bias in the epilogue: the same products
-        // summed in fp32, in another order than the decode step's GEMVs
-        // (512 rows: 318 us as exact-order GEMVs, 35 us here).
+        // matrix cores, scale and bias in the epilogue: the same products as
+        // the decode step's GEMVs, summed in another order and no further from
+        // exact (512 rows: 318 us as exact-order GEMVs, 37 us here).
         check_hip(launch_gather_text_rows(m_.text_embedding_, text_ids, cfg_.text_vocab, rows, H, w.normalized,
                                           stream_),
                   "gather prompt text embeddings");
